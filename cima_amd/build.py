@@ -3,6 +3,7 @@
 Produces, in ``cima_amd/lib/``:
   cima_gemv_a/b/c.hsaco  gfx950 code objects (hipcc --genco): decode GEMVs,
   cima_gemm.hsaco       prefill dequant-GEMMs (MFMA),
+  cima_gemm_wide.hsaco  their 256 x 256 tiles,
   cima_dequant.hsaco    dequant-to-f16 and packed gather,
   cima_decode.hsaco     decode-step support (norm, RoPE, attention, argmax)
   cima_bnb4.hsaco       bitsandbytes NF4/FP4 dequant and decode GEMV
@@ -32,7 +33,7 @@ ARCH = "gfx950"
 SOURCES = {"gemv_a": ("gguf_gemv.hip", ["-DCIMA_GEMV_SET=0"]), "gemv_b": ("gguf_gemv.hip", ["-DCIMA_GEMV_SET=1"]),
            "gemv_c": ("gguf_gemv.hip", ["-DCIMA_GEMV_SET=2"]), "gemm": ("gguf_gemm.hip", []),
            "dequant": ("gguf_dequant.hip", []), "decode": ("decode_ops.hip", []),
-           "bnb4": ("bnb4.hip", [])}
+           "bnb4": ("bnb4.hip", []), "gemm_wide": ("gguf_gemm_wide.hip", [])}
 HSACOS = {name: os.path.join(LIB, f"cima_{name}.hsaco") for name in SOURCES}
 GEMV_OBJECTS = ("gemv_a", "gemv_b", "gemv_c")
 LIBHIP = os.path.join(LIB, "libcima_hip.so")

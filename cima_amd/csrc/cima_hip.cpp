@@ -111,7 +111,7 @@ struct cima_hip_ctx {
     int device = 0;
     int num_cu = 0;
     int max_lds = 0;  // bytes of LDS one workgroup may use
-    hipModule_t modules[7] = {};  // kModuleFiles
+    hipModule_t modules[8] = {};  // kModuleFiles
     bool loaded = false;
     hipStream_t own_stream = nullptr;
     hipStream_t stream = nullptr;
@@ -124,7 +124,7 @@ struct cima_hip_ctx {
     int tune_ring = 0;     // GEMV main loop: 0 = heuristic, 1 = item ring where built, 2 = never
     int tune_ringl = 0;    // stepped ring: 0 = heuristic (8 units per lane), 1 = from 2 units per lane, 2 = never
     int tune_dma = 0;      // direct-to-LDS streaming GEMV: 0 = heuristic, 1 = wherever built, 2 = never
-    int tune_ksplit = 0;   // 16-token GEMM k-split with a slab: 0 = heuristic, 1 = never, 2/4/8 = that many
+    int tune_ksplit = 0;   // prefill GEMM k-split with a slab: 0 = heuristic, 1 = never, 2/4/8 = that many
     int tune_wsplit = 0;   // GEMV rows split over the workgroup's waves: 0 = heuristic, 1 = always, 2 = never
     int tune_nf4_rows = 0;  // NF4 GEMV rows per wave (0 = heuristic, else 1, 2 or 4)
     int tune_nf4_kernel = 0;  // NF4 GEMV: 0 = heuristic, 1 = LDS pair table, 2 = register codebook
@@ -155,11 +155,12 @@ int launch(cima_hip_ctx* ctx, hipFunction_t f, unsigned grid, unsigned block, vo
 }
 
 // code objects: the GEMVs in three (format sets compiled in parallel),
-// the prefill GEMMs, dequant / gather, the decode-step kernels
-enum { MOD_GEMM = 3, MOD_DEQUANT = 4, MOD_DECODE = 5, MOD_BNB4 = 6, NUM_MODULES = 7 };
+// the prefill GEMMs, dequant / gather, the decode-step kernels, and the
+// 256 x 256 prefill tiles (compiled beside the other GEMMs)
+enum { MOD_GEMM = 3, MOD_DEQUANT = 4, MOD_DECODE = 5, MOD_BNB4 = 6, MOD_GEMM_WIDE = 7, NUM_MODULES = 8 };
 const char* const kModuleFiles[NUM_MODULES] = {"cima_gemv_a.hsaco", "cima_gemv_b.hsaco", "cima_gemv_c.hsaco",
                                                "cima_gemm.hsaco",   "cima_dequant.hsaco", "cima_decode.hsaco",
-                                               "cima_bnb4.hsaco"};
+                                               "cima_bnb4.hsaco",   "cima_gemm_wide.hsaco"};
 
 // decode-step kernels (cima_decode.hsaco)
 const char* const kDecodeKernels[] = {
@@ -577,6 +578,13 @@ int cima_hip_init(int device, const char* code_dir, cima_hip_ctx** out) {
                         if (!rc) rc = add(MOD_GEMM, name);
                     }
                 }
+    for (const char* wn : {"q8_0", "q4_0", "q4_1", "q5_0", "q5_1", "q4_k", "q5_k", "q6_k", "iq4_xs", "nf4", "f16w"})
+        for (const char* xt : {"f16", "bf16"})
+            for (const char* yt : {"f32", "f16"}) {
+                char name[96];
+                snprintf(name, sizeof name, "cima_gemm_%s_w256_%s_%s", wn, xt, yt);
+                if (!rc) rc = add(MOD_GEMM_WIDE, name);
+            }
     if (!rc) rc = add(MOD_GEMM, "cima_gemm_ksum_f32");
     if (!rc) rc = add(MOD_GEMM, "cima_gemm_ksum_f16");
     if (!rc) rc = add(MOD_DEQUANT, "cima_stream_read");
@@ -805,33 +813,6 @@ int gemm_check(cima_hip_ctx* ctx, int t, const void* x, const void* w, void* y, 
     return 0;
 }
 
-// Token tile of the fused GEMM (measured on MI355X, Q4_K, bf16 X, cold
-// weights): 16 up to 32 tokens (two 16-token tiles at 33.6 us against 40.2
-// us for one 64-token tile on 14336x4096); 33-128 tokens 32 while that grid
-// fits one workgroup per CU, else 64 (48 tokens: 35.9 against 42.4 us on
-// 14336x4096, 33.6 against 40.0 on 6144x4096; 128 tokens on 14336x4096,
-// 448 workgroups: 61.0 against 44.0); 128 beyond.
-int fused_bn(int m, int n, int num_cu) {
-    if (m <= 32) return 16;
-    if (m <= 128) return (long long)((n + 127) / 128) * ((m + 31) / 32) <= num_cu ? 32 : 64;
-    // 256-token tiles (one workgroup per CU, the weight tile dequantised
-    // once per 256 tokens) where 128-token tiles would need more than 1.5
-    // workgroups per CU and the 256-token grid still fits one round
-    // (measured on MI355X, Q4_K, bf16 X, 14336x4096: 102.2 against 108.8 us
-    // at 512 tokens, 195 against 206 at 1024; a second round of 256-token
-    // workgroups loses: 193 against 165 at 768, and so does a grid that
-    // leaves most CUs idle: 98 against 69 on 6144x4096 at 512)
-    const long long rt = (n + 127) / 128;
-    if (rt * ((m + 255) / 256) <= num_cu && 2 * rt * ((m + 127) / 128) > 3LL * num_cu) return 256;
-    // a weight too narrow for the 128-token grid to fill the CUs takes the
-    // widest register-A tile whose grid still fits one round (measured on
-    // MI355X, Q4_K, bf16 X: 4096x4096 at 256 / 512 tokens 63.0 / 63.6 us
-    // with 128-token tiles, 41.1 / 44.2 with 64-token tiles)
-    if (rt * ((m + 127) / 128) < num_cu && rt * ((m + 63) / 64) <= num_cu)
-        return rt * ((m + 31) / 32) <= num_cu ? 32 : 64;
-    return 128;
-}
-
 // the fused MFMA dequant-GEMM (gguf_gemm.hip) on checked arguments
 // kernel-argument mirror of GemmExt in gguf_gemm.hip (same member order):
 // the bitsandbytes operands; zero for the GGUF formats
@@ -845,76 +826,154 @@ struct GemmExt {
     int ksplit;
 };
 
-// Launches cima_gemm_<fname>_b<BN>[n]_<x>_<y> over Y[m, n] (row stride ldy):
-// the token tile from fused_bn (or the tuning override), 16-token tiles
-// only for k % 128 == 0.
-// Workgroups along k for the 16-token tiles (1 = none), when the caller's
-// slab can hold the partial tiles (S x m x n fp32) and the 128-k stages
-// divide evenly (at least four per split, one per k-split wave).  A grid
-// of 32-row tiles of at most one workgroup per CU is split two ways, a grid
-// of 16-row tiles (the narrow kernels, three or four per CU) four ways at
-// most a quarter workgroup per CU and two ways at most a half.  Measured
-// on MI355X (Q4_K unless noted, bf16 X, cold, us, unsplit -> split): 32
-// tokens: 4096x14336 43.6 -> 30.1 (Q8_0 64.5 -> 48.5), 1024x4096 9.6 ->
-// 8.9, 4096x4096 13.2 -> 13.3; 16 tokens: 6144x4096 15.5 -> 13.9,
-// 1024x4096 9.5 -> 7.9; splitting fuller grids loses (16 tokens:
-// 4096x14336 26.4 -> 27.7, 4096x4096 9.8 -> 12.2, 14336x4096 19.0 -> 23.4).
-int pick_ksplit(const cima_hip_ctx* ctx, int wgs, bool narrow, int m, int n, int k, size_t part_bytes) {
-    const int stages = k / 128;
-    auto fits = [&](int s) { return stages % s == 0 && stages / s >= 4 && (size_t)s * m * n * 4 <= part_bytes; };
-    if (ctx->tune_ksplit == 1) return 1;
-    if (ctx->tune_ksplit > 1) return fits(ctx->tune_ksplit) ? ctx->tune_ksplit : 1;
-    int s = 1;
-    if (!narrow) s = wgs <= ctx->num_cu ? 2 : 1;
-    else s = 4 * wgs <= ctx->num_cu ? 4 : (2 * wgs <= ctx->num_cu ? 2 : 1);
-    while (s > 1 && !fits(s)) s /= 2;
-    return s;
+// The prefill tiles.  b16 / b16n: 16 tokens x 32 / 16 rows (gemm_body_sk16,
+// k % 128 == 0); b32, b64, b128: that many tokens x 64 rows in four k
+// groups (gemm_group; f32 X at 128 tokens: 128 rows, two groups); b256: 128
+// rows x 256 tokens, w256: 256 x 256 (gemm_wide; w256 not for f32 X).
+enum GemmKind { KB16, KB16N, KB32, KB64, KB128, KB256, KW256 };
+struct GemmPlan {
+    GemmKind kind;
+    int ksplit;  // workgroups along k, partial tiles in the slab
+};
+int plan_bm(GemmKind kind, int x_dtype) {
+    switch (kind) {
+    case KB16: return 32;
+    case KB16N: return 16;
+    case KB128: return x_dtype == CIMA_DT_F32 ? 128 : 64;
+    case KB256: return 128;
+    case KW256: return 256;
+    default: return 64;
+    }
+}
+int plan_bn(GemmKind kind) {
+    static const int bn[] = {16, 16, 32, 64, 128, 256, 256};
+    return bn[kind];
 }
 
+// Estimated time (us) of a plan on MI355X: rounds of workgroups over the
+// CUs, each a fixed cost (first loads, staging, output) plus its k stages.
+// The constants are fits to cold runs (Q4_K, bf16 X) of one round at k =
+// 4096 and 14336 -- us per 64-k stage and fixed us: b32 0.20 / 5, b64 0.215
+// / 9.5, b128 0.27 / 13.5, b256 0.81 / 20, w256 1.5 / 20 -- and of the
+// 16-token tiles per 512-k step: 1.5 with one workgroup per CU, 2.05 with
+// two (b16), 0.95 and 1.6 (b16n); `heavy` formats (Q5_K, Q6_K) decode at
+// about 1.7 times that.  A second resident workgroup does not speed the
+// 64-row tiles up (b32 at 14336 rows: 224 workgroups 17.8, 448 34).  The
+// k-split adds the partial tiles' traffic and the summing launch.  Estimated
+// against measured at 14336x4096: 16 / 32 / 64 / 128 / 512 / 2048 tokens 17
+// / 18 / 23 / 31 / 72 / 232 against 17 / 18 / 23 / 31 / 76 / 260; split
+// against unsplit, measured: 4096x14336 at 16 / 100 tokens 19 / 25 and 39 /
+// 111 (Q6_K), 6144x4096 at 32 13.6 / 17, 1024x4096 at 16 9.8 / 9.0 (Q4_K, not
+// split) and 10.9 / 12.3 (Q6_K, split).
+double plan_cost(const cima_hip_ctx* ctx, GemmPlan p, int m, int n, int k, int x_dtype, bool heavy) {
+    const int bm = plan_bm(p.kind, x_dtype), bn = plan_bn(p.kind), cu = ctx->num_cu > 0 ? ctx->num_cu : 1;
+    const double wgs = (double)((n + bm - 1) / bm) * ((m + bn - 1) / bn) * p.ksplit;
+    double t;
+    if (p.kind == KB16 || p.kind == KB16N) {
+        const bool n16 = p.kind == KB16N;
+        const double steps = (k + 511) / 512 / (double)p.ksplit;
+        const double two = (n16 ? 1.6 : 2.05) * (wgs > 2 * cu ? wgs / (2 * cu) : 1.0);
+        t = 1.0 + steps * (heavy ? 1.7 : 1.0) * (wgs <= cu ? (n16 ? 0.95 : 1.5) : two);
+    } else {
+        static const double stage[] = {0, 0, 0.20, 0.215, 0.27, 0.81, 1.5}, fixed[] = {0, 0, 5, 9.5, 13.5, 20, 20};
+        const double wide_f32 = p.kind == KB128 && x_dtype == CIMA_DT_F32 ? 2.0 : 1.0;
+        const double rounds = (double)(((long long)wgs + cu - 1) / cu);
+        t = rounds * (k / 64 / (double)p.ksplit * stage[p.kind] * wide_f32 * (heavy ? 1.7 : 1.0) + fixed[p.kind]);
+    }
+    if (p.ksplit > 1) t += (p.kind <= KB16N ? 6.0 : 3.5) + ((double)p.ksplit * 8 + 4) * m * n / 3e6;
+    return t;
+}
+
+// The cheapest plan by plan_cost: 16-token tiles up to 32 tokens, every
+// wider tile that is at most twice the tokens (a wider one only pads), k
+// split 2 or 4 ways where the slab holds the partial tiles (S x m x n fp32),
+// the stages divide evenly and every split keeps at least eight 64-k
+// stages (four 128-k stages, one per wave, for the 16-token tiles).
+GemmPlan plan_gemm(const cima_hip_ctx* ctx, int m, int n, int k, int x_dtype, bool heavy,
+                   size_t part_bytes) {
+    GemmPlan best{KB32, 1};
+    double best_t = 1e30;
+    auto consider = [&](GemmKind kind) {
+        for (int s : {1, 2, 4, 8}) {
+            if (ctx->tune_ksplit ? s != ctx->tune_ksplit : s == 8) continue;
+            if (s > 1) {
+                const bool sk = kind == KB16 || kind == KB16N;
+                const int stages = sk ? k / 128 : k / 64;
+                if (kind >= KB256 || stages % s || stages / s < (sk ? 4 : 8) || (size_t)s * m * n * 4 > part_bytes) continue;
+            }
+            const double t = plan_cost(ctx, GemmPlan{kind, s}, m, n, k, x_dtype, heavy);
+            if (t < best_t) best_t = t, best = GemmPlan{kind, s};
+        }
+        if (ctx->tune_ksplit > 1 && best_t == 1e30) best = GemmPlan{kind, 1};
+    };
+    const bool sk_ok = k % 128 == 0;
+    if (ctx->tune_gemm_bn) {
+        switch (ctx->tune_gemm_bn) {
+        case 16:
+            if (!sk_ok) consider(KB32);
+            else consider(2LL * ((n + 31) / 32) * ((m + 15) / 16) <= ctx->num_cu ? KB16N : KB16);
+            break;
+        case 32: consider(KB32); break;
+        case 64: consider(KB64); break;
+        case 128: consider(KB128); break;
+        default: consider(KB256);
+        }
+        return best;
+    }
+    if (m <= 32 && sk_ok) {
+        consider(KB16);
+        consider(KB16N);
+    }
+    consider(KB32);
+    if (m > 32) consider(KB64);
+    if (m > 64) consider(KB128);
+    if (m > 128) {
+        consider(KB256);
+        if (x_dtype != CIMA_DT_F32) consider(KW256);
+    }
+    return best;
+}
+
+// Launches the planned tile kernel over Y[m, n] (row stride ldy).  plan_n:
+// the row count the plan is made for (a weight multiplied slice by slice
+// sums every slice in the same order).
 int gemm_launch(cima_hip_ctx* ctx, const char* fname, const void* x, const void* w, void* y, int m, int n, int k,
                 int ldy, int x_dtype, int y_dtype, const GemmExt& gext, const char* api, float* part = nullptr,
-                size_t part_bytes = 0) {
-    // the 16-token tile stages 128 k at a time (32-row weight tiles in
-    // 512-thread workgroups), so it needs k % 128 == 0
-    int bn = fused_bn(m, n, ctx->num_cu);
-    if (ctx->tune_gemm_bn) bn = ctx->tune_gemm_bn;
-    if (bn == 16 && k % 128) bn = 32;
-    // 16-token tiles: 32 rows per 512-thread workgroup, or 16 rows per
-    // 256-thread workgroup (_b16n_) where the 32-row grid, counted over both
-    // of its dimensions, would fill at most half the CUs (measured on MI355X,
-    // Q4_K, bf16 X, 16-row against 32-row tiles, us: m = 16: 1024x4096 9.0 /
-    // 12.9, 4096x4096 9.5 / 13.2, 4096x14336 26.6 / 43.8, 6144x4096 14.8 /
-    // 13.4, 14336x4096 28.9 / 18.7; m = 24-32: 1024x4096 9.2 / 12.8,
-    // 4096x4096 14.7 / 13.5, 4096x14336 44.5 / 43.5)
-    const bool narrow = bn == 16 && 2LL * ((n + 31) / 32) * ((m + 15) / 16) <= ctx->num_cu;
-    const int bm = narrow ? 16 : (bn == 16 ? 32 : 128);  // weight rows per workgroup
+                size_t part_bytes = 0, int plan_n = 0) {
+    const bool heavy = !strcmp(fname, "q5_k") || !strcmp(fname, "q6_k");
+    const GemmPlan p = plan_gemm(ctx, m, plan_n ? plan_n : n, k, x_dtype, heavy, part ? part_bytes : 0);
+    const int bm = plan_bm(p.kind, x_dtype), bn = plan_bn(p.kind), ks = p.ksplit;
+    const bool sk = p.kind == KB16 || p.kind == KB16N;
     static const char* const xn[] = {"f32", "f16", "bf16"};
+    static const char* const kn[] = {"b16", "b16n", "b32", "b64", "b128", "b256", "w256"};
+    // a split group tile writes fp32 partial tiles through its Y
+    const bool part_y = ks > 1 && !sk;
     char name[96];
-    snprintf(name, sizeof name, "cima_gemm_%s_b%d%s_%s_%s", fname, bn, narrow ? "n" : "", xn[x_dtype],
-             y_dtype == CIMA_DT_F32 ? "f32" : "f16");
+    snprintf(name, sizeof name, "cima_gemm_%s_%s_%s_%s", fname, kn[p.kind], xn[x_dtype],
+             y_dtype == CIMA_DT_F32 || part_y ? "f32" : "f16");
     hipFunction_t f;
     if (int rc = get_fn(ctx, name, &f)) return rc;
     const void* xa = x;
     const void* wa = w;
-    void* ya = y;
-    int mm = m, nn = n, kk = k, ld = ldy;
+    void* ya = part_y ? part : y;
+    int mm = m, nn = n, kk = k, ld = part_y ? n : ldy;
     GemmExt ge = gext;
     ge.status = ctx->gemm_xcheck ? ctx->gemm_status : nullptr;
     const unsigned gx = (unsigned)((n + bm - 1) / bm), gy = (unsigned)((m + bn - 1) / bn);
-    const int ks = bn == 16 && part ? pick_ksplit(ctx, (int)(gx * gy), narrow, m, n, k, part_bytes) : 1;
     ge.part = ks > 1 ? part : nullptr;
     ge.ksplit = ks;
     void* args[] = {&xa, &wa, &ya, &mm, &nn, &kk, &ld, &ge};
-    const unsigned threads = bn == 16 && !narrow ? 512 : 256;
-    hipError_t e = hipModuleLaunchKernel(f, gx, gy, (unsigned)ks, threads, 1, 1, 0, ctx->stream, args, nullptr);
+    hipError_t e = hipModuleLaunchKernel(f, gx, gy, (unsigned)ks, p.kind == KB16N ? 256 : 512, 1, 1, 0, ctx->stream,
+                                         args, nullptr);
     if (e != hipSuccess) return hip_fail(e, api);
     if (ks == 1) return 0;
     // the partial tiles, summed in a fixed order into Y
     hipFunction_t fs;
     if (int rc = get_fn(ctx, y_dtype == CIMA_DT_F32 ? "cima_gemm_ksum_f32" : "cima_gemm_ksum_f16", &fs)) return rc;
     const float* pa = part;
-    int S = ks;
-    void* sargs[] = {&pa, &ya, &mm, &nn, &ld, &S};
+    int S = ks, ldo = ldy;
+    void* yo = y;
+    void* sargs[] = {&pa, &yo, &mm, &nn, &ldo, &S};
     const long long outs = (long long)m * n;
     return launch(ctx, fs, (unsigned)((outs + 255) / 256), 256, sargs, api);
 }
@@ -950,7 +1009,7 @@ int cima_hip_gguf_gemm_slab(cima_hip_ctx* ctx, int t, const void* x, const void*
     if (slab_bytes && (!slab || !aligned(slab, 256)))
         return fail(CIMA_E_INVALID, "%s: slab must be a non-null 256-byte aligned device pointer", api);
     // the fused kernels dequantise W tile by tile; the slab holds the
-    // partial tiles when a narrow weight is split along k at 16 tokens
+    // partial tiles when a narrow weight is split along k
     return gemm_launch(ctx, F->name, x, w, y, m, n, k, ldy, x_dtype, y_dtype, GemmExt{}, api,
                        slab_bytes ? static_cast<float*>(slab) : nullptr, (size_t)slab_bytes);
 }
@@ -1553,7 +1612,7 @@ int cima_hip_nf4_gemm_slab(cima_hip_ctx* ctx, const void* x, const void* packed,
             return rc;
         void* ys = static_cast<uint8_t*>(y) + (size_t)r0 * yes;
         if (!small) {
-            if (int rc = gemm_launch(ctx, "f16w", x, slab, ys, m, nr, k, n, x_dtype, y_dtype, GemmExt{}, api))
+            if (int rc = gemm_launch(ctx, "f16w", x, slab, ys, m, nr, k, n, x_dtype, y_dtype, GemmExt{}, api, nullptr, 0, n))
                 return rc;
         } else {
             const void* xa = x;

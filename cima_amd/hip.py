@@ -27,7 +27,7 @@ LIBHIP = os.path.join(LIB_DIR, "libcima_hip.so")
 # the gfx950 code objects cima_hip_init loads (names as cima_amd/build.py
 # writes them)
 CODE_OBJECTS = [os.path.join(LIB_DIR, f"cima_{n}.hsaco")
-                for n in ("gemv_a", "gemv_b", "gemv_c", "gemm", "dequant", "decode", "bnb4")]
+                for n in ("gemv_a", "gemv_b", "gemv_c", "gemm", "dequant", "decode", "bnb4", "gemm_wide")]
 
 # declared in include/cima_hip.h, in order
 EXPORTS = (

@@ -140,10 +140,8 @@ int cima_hip_gemm_status(cima_hip_ctx* ctx, unsigned int* flags, int clear);
 
 /* Prefill GEMM tuning (no counterpart in the reference): token-tile width
  * (16, 32, 64, 128 or 256) for later gguf_gemm calls; 0 = the built-in
- * choice (16 up to 32 tokens; 32 up to 128 while that grid has at most one
- * workgroup per CU, else 64; beyond, 256 where 128-token tiles would need
- * more than 1.5 workgroups per CU and 256-token tiles fit one per CU, else
- * 128). */
+ * choice: the tile, and with a slab the split along k, of the least
+ * estimated time for the shape (plan_gemm in cima_hip.cpp). */
 int cima_hip_set_gemm_tile(cima_hip_ctx* ctx, int tokens);
 
 /* Fused dequant-GEMV: replaces CudaCtx::gguf_gemv (src/cuda.rs:2161-2220).
@@ -192,8 +190,8 @@ int cima_hip_gguf_gemv_swiglu(cima_hip_ctx* ctx, int ggml_type, const void* x,
  * lin_gemm (src/models/transformer.rs:618-655): gguf_dequant of W into an
  * f16 slab (src/cuda.rs:2285) followed by gemm_f16 / gemm_strided_out
  * (src/cuda.rs:2468-2570), with no slab -- each workgroup dequantises its
- * W tile, bit-exact f16, into LDS (128-token tiles) or straight into the
- * MFMA operand registers (up to 64 tokens), and multiplies with f16 MFMA,
+ * W tile, bit-exact f16, into LDS (256-token tiles) or straight into the
+ * MFMA operand registers (up to 128 tokens), and multiplies with f16 MFMA,
  * fp32 accumulate.  x_dtype: CIMA_DT_F32, CIMA_DT_F16 or CIMA_DT_BF16,
  * converted to f16 -- exact for bf16 of 2^-17 <= |x| < 65536; beyond,
  * values overflow to +-inf and below may lose bits as f16 subnormals, which
@@ -210,12 +208,12 @@ int cima_hip_gguf_gemm(cima_hip_ctx* ctx, int ggml_type, const void* x, const vo
  * slab + gemm_dispatch (src/cuda.rs:2285-2320, 2468-2541) runs here as the
  * fused MFMA kernels of cima_hip_gguf_gemm: W is dequantised tile by tile
  * and never expanded, and any slab size, 0 included, works.  No library
- * GEMM is involved.  At up to 32 tokens a weight too narrow to fill the
- * CUs is split along k over more workgroups, with the S partial tiles
- * (S x m x n fp32, S = 2 or 4) in the slab (256-byte aligned) and summed
- * into Y in a fixed order by a second launch; without room in the slab
- * the call runs unsplit.  The slab's contents are then scratch: calls that
- * share a slab must not overlap. */
+ * GEMM is involved.  Where a weight is too narrow to fill the CUs (tiles of
+ * up to 128 tokens) it is split along k over more workgroups, with the S
+ * partial tiles (S x m x n fp32, S = 2 or 4) in the slab (256-byte aligned)
+ * and summed into Y in a fixed order by a second launch; without room in
+ * the slab the call runs unsplit.  The slab's contents are then scratch:
+ * calls that share a slab must not overlap. */
 int cima_hip_gguf_gemm_slab(cima_hip_ctx* ctx, int ggml_type, const void* x, const void* w, void* y,
                             int m, int n, int k, int ldy, int x_dtype, int y_dtype, void* slab,
                             unsigned long long slab_bytes);
