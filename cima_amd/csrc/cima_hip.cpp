@@ -1084,6 +1084,9 @@ int attn_dim_ok(int dim) { return dim == 64 || dim == 128; }
 // positions per attention chunk the kernels stage at most (ATT_MAX_CSZ)
 const int kAttMaxChunk = 256;
 
+// threads of cima_attn_reduce_d<dim> (ATT_MERGE_T in decode_ops.hip)
+const int kAttMergeThreads = 1024;
+
 // query heads per workgroup of cima_attn_decode_d<dim>_c<cp> (AT_GMAX in
 // decode_ops.hip; 4 cp threads, chunks of up to cp positions) and its LDS
 // bytes (sizeof AttnLds2<dim, cp>)
@@ -1181,7 +1184,7 @@ int cima_hip_attn_reduce(cima_hip_ctx* ctx, const float* part, void* out, int q_
     char name[48];
     snprintf(name, sizeof name, "cima_attn_reduce_d%d", dim);
     void* args[] = {&part, &out, &csz, &n_chunks, &seq, &max_seq, &window, &pos_dev};
-    return launch_named(ctx, name, (unsigned)q_heads, 256, args, api);
+    return launch_named(ctx, name, (unsigned)q_heads, kAttMergeThreads, args, api);
 }
 
 int cima_hip_attn_decode_noalloc(cima_hip_ctx* ctx, const void* q, const void* kc, const void* vc, void* out,
@@ -1285,6 +1288,18 @@ int cima_hip_decode_step(cima_hip_ctx* ctx, const cima_decoder* d) {
     if (csz > kAttMaxChunk) return fail(CIMA_E_INVALID, "%s: attn_chunk %d > %d", api, csz, kAttMaxChunk);
     const int nch = (d->max_seq + csz - 1) / csz;
     const float scale = 1.0f / sqrtf((float)hd);
+    // The split partials are merged by a launch of their own (into the q
+    // part of qkv, which the attention launch has consumed) rather than in
+    // every workgroup of the o projection where the partials of a full cache
+    // pass 128 KB: each of the projection's workgroups reads all live ones.
+    // Measured on MI355X, us per step, merged inside / apart: Llama-3-8B
+    // layers (4 of them, Q4_K) at position 10 of 1024 (133 KB) 217 / 194, 1000
+    // of 2048 226 / 198, 10 of 8192 245 / 211, 8000 of 8192 373 / 220;
+    // Qwen2.5-0.5B (24 layers, Q8_0) at 10 of 4096 (118 KB) 617 / 623, 2047
+    // of 4096 631 / 652, 10 of 8192 620 / 628, 8000 of 8192 798 / 666.
+    // Rows of q past 16384 elements keep the fused launch and its LDS limit.
+    const bool merge_apart = (size_t)d->q_heads * nch * (hd + 2) * 4 > (128u << 10) && qd <= 16384;
+    if (!aligned(d->part, 8)) return fail(CIMA_E_INVALID, "%s: partials must be 8-byte aligned", api);
     const void* head = d->head ? d->head : d->embed;
     const int head_type = d->head ? d->head_type : d->embed_type;
     // enqueue_decode_device (src/models/transformer.rs:1440-1461)
@@ -1321,9 +1336,17 @@ int cima_hip_decode_step(cima_hip_ctx* ctx, const cima_decoder* d) {
                                 csz, nch, d->rope_theta, scale, L.window, d->pos, api))
             return rc;
         // merge of the partials -> o projection + residual (:1161-1238)
-        if (int rc = cima_hip_attn_gguf_gemv(ctx, ty(L.type_o), d->part, d->q_heads, hd, csz, nch, d->max_seq,
-                                             L.window, d->pos, L.wo, nullptr, d->x, d->hidden, 1))
+        if (merge_apart) {
+            if (int rc = cima_hip_attn_reduce(ctx, d->part, d->qkv, d->q_heads, hd, csz, nch, 1, d->max_seq, L.window,
+                                              d->pos))
+                return rc;
+            if (int rc = cima_hip_gguf_gemv(ctx, ty(L.type_o), d->qkv, L.wo, nullptr, d->x, d->hidden, qd, 1,
+                                            CIMA_DT_F16))
+                return rc;
+        } else if (int rc = cima_hip_attn_gguf_gemv(ctx, ty(L.type_o), d->part, d->q_heads, hd, csz, nch, d->max_seq,
+                                                    L.window, d->pos, L.wo, nullptr, d->x, d->hidden, 1)) {
             return rc;
+        }
         // rmsnorm -> gate|up SwiGLU -> down + residual (:1240-1260)
         if (!L.w_up) {
             if (int rc = cima_hip_rmsnorm_gguf_gemv(ctx, ty(L.type_gate), d->x, L.ffn_norm, d->rms_eps, L.w_gate_up,
