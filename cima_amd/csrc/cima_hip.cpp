@@ -1084,6 +1084,9 @@ int attn_dim_ok(int dim) { return dim == 64 || dim == 128; }
 // positions per attention chunk the kernels stage at most (ATT_MAX_CSZ)
 const int kAttMaxChunk = 256;
 
+// heads per workgroup of cima_rope_f16 (ROPE_HEADS in decode_ops.hip)
+const int kRopeHeads = 16;
+
 // threads of cima_attn_reduce_d<dim> (ATT_MERGE_T in decode_ops.hip)
 const int kAttMergeThreads = 1024;
 
@@ -1141,7 +1144,8 @@ int cima_hip_rope(cima_hip_ctx* ctx, void* x, int rows, int heads, int dim, int 
     if (rows == 0) return 0;
     if (!x) return fail(CIMA_E_INVALID, "%s: null x", api);
     void* args[] = {&x, &heads, &dim, &pos0, &theta, &nfreqs, &pos_dev};
-    return launch_named(ctx, "cima_rope_f16", (unsigned)(rows * heads), 64, args, api);
+    const long long hgs = (heads + kRopeHeads - 1) / kRopeHeads;
+    return launch_named(ctx, "cima_rope_f16", (unsigned)(rows * hgs), 256, args, api);
 }
 
 int cima_hip_kv_append(cima_hip_ctx* ctx, const void* k, const void* v, void* kc, void* vc, int rows, int kv_heads,
