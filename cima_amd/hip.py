@@ -142,28 +142,50 @@ def load_library(path: str = LIBHIP) -> ctypes.CDLL:
     return L
 
 
+_raw_stream = None
+_act_types: dict = {}
+_gemm_types: dict = {}
+
+
+def _torch_names() -> None:
+    """torch's raw-stream query and the activation types, looked up once
+    (torch is imported only by programs that pass tensors)."""
+    global _raw_stream
+    import torch
+
+    _act_types.update({torch.float32: gguf.DT_F32, torch.float16: gguf.DT_F16})
+    _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+        lambda device: torch.cuda.current_stream(device).cuda_stream)
+
+
+# Every call passes four to six operands through _ptr and most read x's type:
+# they are written for the tensor case, one attribute each and no second
+# look at the argument's class.  Small GEMVs are bound by this Python side:
+# with the raw stream query 7.2 -> 5.9 us a call (Q8_0 4864 x 896, whose
+# kernel takes 3.4 us).
 def _ptr(a) -> Optional[int]:
-    if a is None or (isinstance(a, int) and a == 0):
+    if a is None:
         return None
-    if isinstance(a, int):
-        return a
-    if hasattr(a, "data_ptr"):
-        if not a.is_cuda:
-            raise EngineError("hip", E_INVALID, "tensor argument is not on a HIP device")
-        if not a.is_contiguous():
-            raise EngineError("hip", E_INVALID, "tensor argument is not contiguous")
-        return a.data_ptr()
-    raise TypeError(f"expected a device pointer or a torch tensor, got {type(a)!r}")
+    try:
+        on_device, contiguous = a.is_cuda, a.is_contiguous
+    except AttributeError:
+        if isinstance(a, int):
+            return a or None
+        raise TypeError(f"expected a device pointer or a torch tensor, got {type(a)!r}") from None
+    if not on_device:
+        raise EngineError("hip", E_INVALID, "tensor argument is not on a HIP device")
+    if not contiguous():
+        raise EngineError("hip", E_INVALID, "tensor argument is not contiguous")
+    return a.data_ptr()
 
 
 def _act_of(t) -> int:
-    import torch
-
-    if t.dtype == torch.float32:
-        return gguf.DT_F32
-    if t.dtype == torch.float16:
-        return gguf.DT_F16
-    raise EngineError("hip", E_INVALID, f"activation dtype {t.dtype} is not float32 or float16")
+    if not _act_types:
+        _torch_names()
+    act = _act_types.get(t.dtype)
+    if act is None:
+        raise EngineError("hip", E_INVALID, f"activation dtype {t.dtype} is not float32 or float16")
+    return act
 
 
 class HipCtx:
@@ -213,9 +235,9 @@ class HipCtx:
     def use_torch_stream(self) -> None:
         """Launch on torch's current stream of this device (ordered with
         torch's own kernels there)."""
-        import torch
-
-        self.set_stream(torch.cuda.current_stream(self.device).cuda_stream)
+        if _raw_stream is None:
+            _torch_names()
+        self._check(self.lib.cima_hip_set_stream(self.handle, _raw_stream(self.device)))
 
     def sync(self) -> None:
         self._check(self.lib.cima_hip_sync(self.handle))
@@ -275,10 +297,12 @@ class HipCtx:
         def dt(t, default):
             if t is not None:
                 return t
-            import torch
+            if not _gemm_types:
+                import torch
 
-            return {torch.float32: gguf.DT_F32, torch.float16: gguf.DT_F16,
-                    torch.bfloat16: gguf.DT_BF16}.get(getattr(x if default == "x" else y, "dtype", None), gguf.DT_F32)
+                _gemm_types.update({torch.float32: gguf.DT_F32, torch.float16: gguf.DT_F16,
+                                    torch.bfloat16: gguf.DT_BF16})
+            return _gemm_types.get(getattr(x if default == "x" else y, "dtype", None), gguf.DT_F32)
         xd = dt(x_dtype, "x") if hasattr(x, "dtype") or x_dtype is not None else gguf.DT_F32
         yd = dt(y_dtype, "y") if hasattr(y, "dtype") or y_dtype is not None else gguf.DT_F32
         return xd, yd
