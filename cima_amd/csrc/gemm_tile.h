@@ -68,7 +68,9 @@ DEV void store4(void* y, float4_t o, int tok, int row, int m, int n, int ldy, bo
 template <typename D, int XT, int YT, int TB, int RG, int KG, int PFW>
 DEV void gemm_group(const void* __restrict__ x, const uint8_t* __restrict__ w, void* __restrict__ y, int m,
                           int n, int k, int ldy, const GemmExt& ext) {
-    constexpr int RA = 1;                        // 32-row tiles per wave
+    // 32-row tiles per wave: one; more rows go to more workgroups (two leave
+    // too few registers for two waves per SIMD)
+    constexpr int RA = 1;
     constexpr int BK = 64, KP = BK + 8;          // stage depth and LDS pitch (halves)
     constexpr int T = 32 * TB, BM = 32 * RA * RG;
     constexpr int NT = 64 * RG;                  // threads of a k group
@@ -254,7 +256,6 @@ DEV void gemm_group(const void* __restrict__ x, const uint8_t* __restrict__ w, v
     // split along k: Y is the partial tiles [ksplit][m][ldy], fp32, summed
     // by cima_gemm_ksum_*
     void* yz = static_cast<uint8_t*>(y) + (size_t)blockIdx.z * m * ldy * (YT == XT_F32 ? 4 : 2);
-    // split along k: Y is the partial tiles [ksplit][m][ldy], fp32
     static_for<TB>([&](auto B) INL {
         const int tok = t0 + 32 * B + (lane & 31);
         static_for<4>([&](auto VV) INL {

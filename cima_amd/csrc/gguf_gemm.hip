@@ -137,10 +137,10 @@ __device__ void gemm_body_sk16(const void* __restrict__ x, const uint8_t* __rest
     xscan.finish(x, ext.status);
 }
 
-
 // Raw weights in flight per wave of the group tiles: two stages, and at 64
 // tokens four where the raw sub-block is small (measured on MI355X, Q4_K,
-// 14336x4096 at 64 tokens: 23.2 against 29 us).
+// 14336x4096 at 64 tokens: 23.2 us; two stages at four waves per SIMD
+// instead spill registers: 38.8 us).
 template <typename D, int BN>
 constexpr int group_pf() { return BN == 64 && sizeof(typename D::Raw) <= 48 ? 4 : 2; }
 // Waves per SIMD asked for: 32-token tiles fit four in 128 registers except

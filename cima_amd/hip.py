@@ -318,8 +318,8 @@ class HipCtx:
                        ldy: Optional[int] = None, x_dtype: Optional[int] = None,
                        y_dtype: Optional[int] = None) -> None:
         """The same product through the reference's lin_gemm signature (the
-        engine's scratch slab is accepted and left untouched: the fused
-        kernels never expand W)."""
+        engine's scratch slab is accepted: the fused kernels never expand W
+        into it, but may keep partial tiles of a split along k there)."""
         xd, yd = self._gemm_dtypes(x, y, x_dtype, y_dtype)
         if slab_bytes is None:
             slab_bytes = 0 if slab is None else slab.numel() * slab.element_size()

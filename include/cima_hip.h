@@ -54,10 +54,10 @@ typedef struct cima_hip_ctx cima_hip_ctx;
 
 /* Context creation: replaces CudaCtx::init (src/cuda.rs:691-908) -- device
  * selection, one non-blocking stream, then loading the prebuilt gfx950 code
- * objects (cima_gemv_a/b/c.hsaco, cima_gemm.hsaco, cima_dequant.hsaco,
- * cima_decode.hsaco) with
- * hipModuleLoad and resolving every kernel (the reference JIT-compiles with
- * NVRTC and resolves its KernelSet, src/cuda.rs:808-877).
+ * objects (cima_gemv_a/b/c.hsaco, cima_gemm.hsaco, cima_gemm_wide.hsaco,
+ * cima_dequant.hsaco, cima_decode.hsaco, cima_bnb4.hsaco) with hipModuleLoad
+ * and resolving every kernel (the reference JIT-compiles with NVRTC and
+ * resolves its KernelSet, src/cuda.rs:808-877).
  * code_dir: directory holding the code objects, or NULL for the directory
  * of this library. */
 int cima_hip_init(int device, const char* code_dir, cima_hip_ctx** out);
