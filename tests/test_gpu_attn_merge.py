@@ -68,3 +68,23 @@ def test_decode_step_merging_apart(hip, head_dim, q_heads, kv_heads, max_seq, ch
         want = want.astype(np.float64)
         assert np.linalg.norm(got - want) / np.linalg.norm(want) <= 2.0 * np.sqrt(2) * 1e-3
         assert d.position() == ctx_len + 1
+
+
+def test_merging_apart_replays_as_eager(hip):
+    """The step with its merge launch, captured once: every replay equals an
+    eager step of a second decoder in the same state."""
+    cfg = DecoderConfig(n_layers=2, hidden=512, q_heads=16, kv_heads=4, head_dim=64, ffn=512, vocab=1000, max_seq=2048,
+                        attn_chunk=64)
+    m = synthetic_model(cfg, seed=8)
+    eager, graph = DeviceDecoder(hip, m), DeviceDecoder(hip, m)
+    for d in (eager, graph):
+        for i in range(cfg.n_layers):
+            d.load_kv(i, *synthetic_kv(cfg, i, 700))
+        d.set_state(3, 700)
+    graph.capture()
+    for s in range(4):
+        eager.step()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(eager.logits, graph.logits), s
+        assert eager.token() == graph.token() and graph.position() == 701 + s
