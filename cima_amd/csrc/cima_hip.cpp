@@ -120,7 +120,8 @@ struct cima_hip_ctx {
     int tune_rows = 0;
     int tune_lpr = 0;
     int tune_wgs = 0;  // workgroups per CU of the persistent grid (0 = built-in default)
-    int tune_gemm_bn = 0;  // prefill GEMM token tile (0 = smallest built one covering m)
+    int tune_gemm_bn = 0;  // prefill GEMM token tile (0 = planned)
+    int tune_gemm_kind = -1;  // prefill GEMM tile kind (-1 = by tune_gemm_bn, else planned)
     int tune_ring = 0;     // GEMV main loop: 0 = heuristic, 1 = item ring where built, 2 = never
     int tune_ringl = 0;    // stepped ring: 0 = heuristic (8 units per lane), 1 = from 2 units per lane, 2 = never
     int tune_dma = 0;      // direct-to-LDS streaming GEMV: 0 = heuristic, 1 = wherever built, 2 = never
@@ -624,7 +625,7 @@ int cima_hip_init(int device, const char* code_dir, cima_hip_ctx** out) {
     if (const char* s = getenv("CIMA_GEMV_RINGL")) ctx->tune_ringl = atoi(s);
     if (const char* s = getenv("CIMA_GEMV_DMA")) ctx->tune_dma = atoi(s);
     if (const char* s = getenv("CIMA_GEMM_XCHECK")) ctx->gemm_xcheck = atoi(s) != 0;
-    if (const char* s = getenv("CIMA_GEMM_KSPLIT")) ctx->tune_ksplit = atoi(s);
+    if (const char* s = getenv("CIMA_GEMM_KSPLIT")) ctx->tune_ksplit = std::max(atoi(s), 0);
     if (const char* s = getenv("CIMA_GEMV_WSPLIT")) ctx->tune_wsplit = atoi(s);
     if (er || el) {
         if (int r = cima_hip_set_gemv_tuning(ctx, er, el)) {
@@ -814,7 +815,7 @@ int gemm_check(cima_hip_ctx* ctx, int t, const void* x, const void* w, void* y, 
 }
 
 // the fused MFMA dequant-GEMM (gguf_gemm.hip) on checked arguments
-// kernel-argument mirror of GemmExt in gguf_gemm.hip (same member order):
+// kernel-argument mirror of GemmExt in gemm_decode.h (same member order):
 // the bitsandbytes operands; zero for the GGUF formats
 struct GemmExt {
     const float* absmax;
@@ -865,8 +866,8 @@ int plan_bn(GemmKind kind) {
 // against unsplit, measured: 4096x14336 at 16 / 100 tokens 19 / 25 and 39 /
 // 111 (Q6_K), 6144x4096 at 32 13.6 / 17, 1024x4096 at 16 9.8 / 9.0 (Q4_K, not
 // split) and 10.9 / 12.3 (Q6_K, split).
-double plan_cost(const cima_hip_ctx* ctx, GemmPlan p, int m, int n, int k, int x_dtype, bool heavy) {
-    const int bm = plan_bm(p.kind, x_dtype), bn = plan_bn(p.kind), cu = ctx->num_cu > 0 ? ctx->num_cu : 1;
+double plan_cost(int cu, GemmPlan p, int m, int n, int k, int x_dtype, bool heavy) {
+    const int bm = plan_bm(p.kind, x_dtype), bn = plan_bn(p.kind);
     const double wgs = (double)((n + bm - 1) / bm) * ((m + bn - 1) / bn) * p.ksplit;
     double t;
     if (p.kind == KB16 || p.kind == KB16N) {
@@ -884,34 +885,51 @@ double plan_cost(const cima_hip_ctx* ctx, GemmPlan p, int m, int n, int k, int x
     return t;
 }
 
+// Overrides of the plan (cima_hip_set_gemm_tile, cima_hip_set_gemm_plan,
+// CIMA_GEMM_KSPLIT).
+struct GemmTune {
+    int bn = 0;      // token tile, 0 = planned
+    int kind = -1;   // GemmKind, before bn; -1 = none
+    int ksplit = 0;  // 0 = planned, 1 = none, else this many where they divide and fit
+};
+
 // The cheapest plan by plan_cost: 16-token tiles up to 32 tokens, every
 // wider tile that is at most twice the tokens (a wider one only pads), k
 // split 2 or 4 ways where the slab holds the partial tiles (S x m x n fp32),
 // the stages divide evenly and every split keeps at least eight 64-k
 // stages (four 128-k stages, one per wave, for the 16-token tiles).
-GemmPlan plan_gemm(const cima_hip_ctx* ctx, int m, int n, int k, int x_dtype, bool heavy,
-                   size_t part_bytes) {
+GemmPlan plan_gemm(const GemmTune& tune, int num_cu, int m, int n, int k, int x_dtype, bool heavy, size_t part_bytes) {
+    const int cu = num_cu > 0 ? num_cu : 1;
     GemmPlan best{KB32, 1};
     double best_t = 1e30;
     auto consider = [&](GemmKind kind) {
-        for (int s : {1, 2, 4, 8}) {
-            if (ctx->tune_ksplit ? s != ctx->tune_ksplit : s == 8) continue;
-            if (s > 1) {
-                const bool sk = kind == KB16 || kind == KB16N;
-                const int stages = sk ? k / 128 : k / 64;
-                if (kind >= KB256 || stages % s || stages / s < (sk ? 4 : 8) || (size_t)s * m * n * 4 > part_bytes) continue;
+        const bool sk = kind == KB16 || kind == KB16N;
+        const int stages = sk ? k / 128 : k / 64;
+        for (int s : {1, 2, 4}) {
+            if (tune.ksplit && s > 1) break;
+            if (tune.ksplit) s = tune.ksplit;
+            if (s > 1 &&
+                (kind >= KB256 || stages % s || stages / s < (sk ? 4 : 8) || (size_t)s * m * n * 4 > part_bytes)) {
+                if (!tune.ksplit) continue;
+                s = 1;
             }
-            const double t = plan_cost(ctx, GemmPlan{kind, s}, m, n, k, x_dtype, heavy);
+            const double t = plan_cost(cu, GemmPlan{kind, s}, m, n, k, x_dtype, heavy);
             if (t < best_t) best_t = t, best = GemmPlan{kind, s};
         }
-        if (ctx->tune_ksplit > 1 && best_t == 1e30) best = GemmPlan{kind, 1};
     };
     const bool sk_ok = k % 128 == 0;
-    if (ctx->tune_gemm_bn) {
-        switch (ctx->tune_gemm_bn) {
+    if (tune.kind >= 0) {
+        GemmKind kind = (GemmKind)tune.kind;
+        if ((kind == KB16 || kind == KB16N) && !sk_ok) kind = KB32;
+        if (kind == KW256 && x_dtype == CIMA_DT_F32) kind = KB256;
+        consider(kind);
+        return best;
+    }
+    if (tune.bn) {
+        switch (tune.bn) {
         case 16:
             if (!sk_ok) consider(KB32);
-            else consider(2LL * ((n + 31) / 32) * ((m + 15) / 16) <= ctx->num_cu ? KB16N : KB16);
+            else consider(2LL * ((n + 31) / 32) * ((m + 15) / 16) <= cu ? KB16N : KB16);
             break;
         case 32: consider(KB32); break;
         case 64: consider(KB64); break;
@@ -934,14 +952,17 @@ GemmPlan plan_gemm(const cima_hip_ctx* ctx, int m, int n, int k, int x_dtype, bo
     return best;
 }
 
+// formats whose decoding plan_cost charges for
+bool heavy_fmt(const char* name) { return !strcmp(name, "q5_k") || !strcmp(name, "q6_k"); }
+
 // Launches the planned tile kernel over Y[m, n] (row stride ldy).  plan_n:
 // the row count the plan is made for (a weight multiplied slice by slice
 // sums every slice in the same order).
 int gemm_launch(cima_hip_ctx* ctx, const char* fname, const void* x, const void* w, void* y, int m, int n, int k,
                 int ldy, int x_dtype, int y_dtype, const GemmExt& gext, const char* api, float* part = nullptr,
                 size_t part_bytes = 0, int plan_n = 0) {
-    const bool heavy = !strcmp(fname, "q5_k") || !strcmp(fname, "q6_k");
-    const GemmPlan p = plan_gemm(ctx, m, plan_n ? plan_n : n, k, x_dtype, heavy, part ? part_bytes : 0);
+    const GemmPlan p = plan_gemm(GemmTune{ctx->tune_gemm_bn, ctx->tune_gemm_kind, ctx->tune_ksplit}, ctx->num_cu, m,
+                                 plan_n ? plan_n : n, k, x_dtype, heavy_fmt(fname), part ? part_bytes : 0);
     const int bm = plan_bm(p.kind, x_dtype), bn = plan_bn(p.kind), ks = p.ksplit;
     const bool sk = p.kind == KB16 || p.kind == KB16N;
     static const char* const xn[] = {"f32", "f16", "bf16"};
@@ -1012,6 +1033,33 @@ int cima_hip_gguf_gemm_slab(cima_hip_ctx* ctx, int t, const void* x, const void*
     // partial tiles when a narrow weight is split along k
     return gemm_launch(ctx, F->name, x, w, y, m, n, k, ldy, x_dtype, y_dtype, GemmExt{}, api,
                        slab_bytes ? static_cast<float*>(slab) : nullptr, (size_t)slab_bytes);
+}
+
+int cima_hip_set_gemm_plan(cima_hip_ctx* ctx, int rows, int tokens, int ksplit) {
+    const char* api = "cima_hip_set_gemm_plan";
+    if (!ctx) return fail(CIMA_E_NOT_INIT, "%s: null context", api);
+    int kind = -1;
+    for (int i = KB16; i <= KW256; i++)
+        if (rows == plan_bm((GemmKind)i, CIMA_DT_F16) && tokens == plan_bn((GemmKind)i)) kind = i;
+    if (kind < 0 && (rows || tokens)) return fail(CIMA_E_INVALID, "%s: no %d x %d tile is built", api, rows, tokens);
+    if (ksplit < 0 || ksplit > 8 || (ksplit & (ksplit - 1)))
+        return fail(CIMA_E_INVALID, "%s: ksplit %d is not 0, 1, 2, 4 or 8", api, ksplit);
+    ctx->tune_gemm_kind = kind;
+    ctx->tune_ksplit = ksplit;
+    return 0;
+}
+
+int cima_hip_gemm_plan(int num_cu, int t, int m, int n, int k, int x_dtype, unsigned long long slab_bytes, int* rows,
+                       int* tokens, int* ksplit) {
+    const char* api = "cima_hip_gemm_plan";
+    const Fmt* F = t ? fmt_of(t) : nullptr;
+    if (t && !F) return fail(CIMA_E_FORMAT, "%s: ggml type %d is not a supported GGUF block format", api, t);
+    if (num_cu <= 0 || m <= 0 || n <= 0 || k <= 0 || k % 64 || x_dtype < CIMA_DT_F32 || x_dtype > CIMA_DT_BF16)
+        return fail(CIMA_E_INVALID, "%s: num_cu=%d m=%d n=%d k=%d x_dtype=%d", api, num_cu, m, n, k, x_dtype);
+    if (!rows || !tokens || !ksplit) return fail(CIMA_E_INVALID, "%s: null pointer", api);
+    const GemmPlan p = plan_gemm(GemmTune{}, num_cu, m, n, k, x_dtype, F && heavy_fmt(F->name), (size_t)slab_bytes);
+    *rows = plan_bm(p.kind, x_dtype), *tokens = plan_bn(p.kind), *ksplit = p.ksplit;
+    return 0;
 }
 
 

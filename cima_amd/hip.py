@@ -35,6 +35,7 @@ EXPORTS = (
     "cima_hip_get_stream",
     "cima_hip_sync", "cima_hip_last_error", "cima_hip_is_fatal", "cima_hip_num_cu", "cima_hip_set_gemv_tuning",
     "cima_hip_set_gemv_dma", "cima_hip_set_gemv_wsplit", "cima_hip_set_gemv_grid", "cima_hip_gemm_status", "cima_hip_set_gemm_tile",
+    "cima_hip_set_gemm_plan", "cima_hip_gemm_plan",
     "cima_hip_gguf_gemv", "cima_hip_rmsnorm_gguf_gemv",
     "cima_hip_gguf_gemv_swiglu", "cima_hip_gguf_gemm", "cima_hip_gguf_gemm_slab", "cima_hip_gguf_dequant", "cima_hip_gguf_gather",
     "cima_hip_rmsnorm", "cima_hip_rope", "cima_hip_kv_append", "cima_hip_attn_decode_split", "cima_hip_attn_reduce",
@@ -107,6 +108,8 @@ def load_library(path: str = LIBHIP) -> ctypes.CDLL:
     L.cima_hip_gemm_status.argtypes = [P, ctypes.POINTER(ctypes.c_uint), I]
     L.cima_hip_set_gemv_grid.argtypes = [P, I]
     L.cima_hip_set_gemm_tile.argtypes = [P, I]
+    L.cima_hip_set_gemm_plan.argtypes = [P, I, I, I]
+    L.cima_hip_gemm_plan.argtypes = [I, I, I, I, I, I, ctypes.c_ulonglong] + [ctypes.POINTER(I)] * 3
     L.cima_hip_gguf_gemv.argtypes = [P, I, P, P, P, P, I, I, I, I]
     F = ctypes.c_float
     L.cima_hip_rmsnorm_gguf_gemv.argtypes = [P, I, P, P, F, P, P, P, I, I, I, I]
@@ -186,6 +189,17 @@ def _act_of(t) -> int:
     if act is None:
         raise EngineError("hip", E_INVALID, f"activation dtype {t.dtype} is not float32 or float16")
     return act
+
+
+def gemm_plan(fmt: int, m: int, n: int, k: int, x_dtype: int, slab_bytes: int = 0, num_cu: int = 256) -> tuple:
+    """(tile rows, tile tokens, split along k) of a prefill product on a device of
+    ``num_cu`` compute units (cima_hip_gemm_plan; ``fmt`` 0: bitsandbytes)."""
+    L = load_library()
+    out = [ctypes.c_int() for _ in range(3)]
+    rc = L.cima_hip_gemm_plan(num_cu, int(fmt), m, n, k, x_dtype, int(slab_bytes), *(ctypes.byref(v) for v in out))
+    if rc:
+        raise EngineError("hip", rc, L.cima_hip_last_error().decode(errors="replace"))
+    return tuple(v.value for v in out)
 
 
 class HipCtx:
@@ -269,6 +283,10 @@ class HipCtx:
     def set_gemm_tile(self, tokens: int = 0) -> None:
         """Prefill GEMM token-tile width (16, 32, 64, 128 or 256; 0 = built-in choice)."""
         self._check(self.lib.cima_hip_set_gemm_tile(self.handle, int(tokens)))
+
+    def set_gemm_plan(self, rows: int = 0, tokens: int = 0, ksplit: int = 0) -> None:
+        """Prefill GEMM tile kind and split along k (cima_hip_set_gemm_plan; 0, 0, 0 = built-in choice)."""
+        self._check(self.lib.cima_hip_set_gemm_plan(self.handle, int(rows), int(tokens), int(ksplit)))
 
     def set_gemv_grid(self, wgs_per_cu: int = 0) -> None:
         """Cap the persistent GEMV grid at this many workgroups per CU (0 = fill)."""

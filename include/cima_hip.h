@@ -144,6 +144,23 @@ int cima_hip_gemm_status(cima_hip_ctx* ctx, unsigned int* flags, int clear);
  * estimated time for the shape (plan_gemm in cima_hip.cpp). */
 int cima_hip_set_gemm_tile(cima_hip_ctx* ctx, int tokens);
 
+/* The same for one tile kind and split (no counterpart in the reference):
+ * rows x tokens of a workgroup's tile -- 16 x 16, 32 x 16, 64 x 32, 64 x 64,
+ * 64 x 128 (128 x 128 for f32 X), 128 x 256 or 256 x 256 -- or 0, 0 for
+ * cima_hip_set_gemm_tile's choice, and the split along k (0 = planned, 1 =
+ * none, 2, 4 or 8 where the stages divide and the slab holds the partial
+ * tiles; never for the 256-token tiles).  Calls a forced tile does not
+ * take run the next one: 64 x 32 where k % 128 != 0, 128 x 256 for f32 X. */
+int cima_hip_set_gemm_plan(cima_hip_ctx* ctx, int rows, int tokens, int ksplit);
+
+/* The plan of a prefill product without overrides (no counterpart in the
+ * reference): tile rows and tokens and the split along k that gguf_gemm
+ * (slab_bytes 0) or gguf_gemm_slab takes on a device of num_cu compute
+ * units.  ggml_type 0: bitsandbytes weights (nf4_gemm_slab, which never
+ * splits).  Needs no device. */
+int cima_hip_gemm_plan(int num_cu, int ggml_type, int m, int n, int k, int x_dtype, unsigned long long slab_bytes,
+                       int* rows, int* tokens, int* ksplit);
+
 /* Fused dequant-GEMV: replaces CudaCtx::gguf_gemv (src/cuda.rs:2161-2220).
  *   y[r] = sum_j W[r, j] * x[j] for r in [0, n), W packed GGUF rows of k
  *   elements (row r at r * storage_bytes(fmt, k)).

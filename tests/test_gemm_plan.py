@@ -1,0 +1,44 @@
+"""The planner of the prefill products, asked without a device (cima_hip_gemm_plan
+on 256 compute units)."""
+import ctypes
+
+import pytest
+
+from cima_amd import gguf, hip
+
+F32, F16, BF16 = gguf.DT_F32, gguf.DT_F16, gguf.DT_BF16
+SLAB = 32 << 20
+TILES = {(16, 16), (32, 16), (64, 32), (64, 64), (64, 128), (128, 128), (128, 256), (256, 256)}
+
+
+@pytest.mark.parametrize("t", [0] + [int(f) for f in gguf.DType])
+@pytest.mark.parametrize("xd", [F32, F16, BF16])
+def test_every_plan_can_run(t, xd):
+    """A built tile, 16-token tiles only for k % 128 == 0, 256 x 256 not for f32
+    X, a split only into ranges the tile takes and the slab holds."""
+    for m in (1, 16, 17, 32, 33, 64, 65, 100, 128, 129, 256, 300, 700, 2048, 5000):
+        for n in (1, 63, 300, 1024, 4096, 14336, 128256):
+            for k in (256, 768, 4096, 14336) + (() if t in (12, 13, 14, 23) else (64, 192, 832)):
+                for slab in (0, 1 << 16, SLAB):
+                    rows, tokens, ks = hip.gemm_plan(t, m, n, k, xd, slab)
+                    assert (rows, tokens) in TILES
+                    assert (rows, tokens) != ((256, 256) if xd == F32 else (128, 128))
+                    assert (rows, tokens) != (64, 128) or xd != F32
+                    assert tokens != 16 or k % 128 == 0
+                    stages, least = (k // 128, 4) if tokens == 16 else (k // 64, 8)
+                    assert ks == 1 or (ks in (2, 4) and tokens <= 128 and stages % ks == 0 and stages // ks >= least
+                                       and 4 * ks * m * n <= slab)
+
+
+def test_refusals():
+    for bad in ((0, 16, 16, 256), (256, 0, 16, 256), (256, 16, 16, 100), (256, 16, 16, -256)):
+        cu, m, n, k = bad
+        with pytest.raises(hip.EngineError):
+            hip.gemm_plan(12, m, n, k, F16, 0, cu)
+    with pytest.raises(hip.EngineError):
+        hip.gemm_plan(99, 16, 16, 256, F16)
+    with pytest.raises(hip.EngineError):
+        hip.gemm_plan(12, 16, 16, 256, 7)
+    L = hip.load_library()
+    assert L.cima_hip_gemm_plan(256, 12, 16, 16, 256, F16, 0, None, None, ctypes.byref(ctypes.c_int())) == hip.E_INVALID
+    assert L.cima_hip_set_gemm_plan(None, 64, 64, 1) == hip.E_NOT_INIT

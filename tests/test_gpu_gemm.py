@@ -116,7 +116,7 @@ def test_gemm_argument_errors(hip):
 
 
 @pytest.mark.parametrize("t", FORMATS, ids=[NAMES[t] for t in FORMATS])
-@pytest.mark.parametrize("bn", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("bn", [16, 32, 64, 128, 256, "256x256"])
 def test_gemm_dequantises_bit_exactly(hip, t, bn):
     """With X the identity, Y = dequant(W)^T: every f16 weight the kernel
     multiplies, read back exactly (an f16 times 1.0, summed with exact
@@ -125,18 +125,22 @@ def test_gemm_dequantises_bit_exactly(hip, t, bn):
     k = 256
     n = 96
     nbytes = n * k // oracle.BLOCK_ELEMS[t] * oracle.BLOCK_BYTES[t]
-    raw = mg.xorshift_bytes(nbytes, seed=0x9E3779B97F4A7C15 + bn)
+    raw = mg.xorshift_bytes(nbytes, seed=0x9E3779B97F4A7C15 + (bn if isinstance(bn, int) else 257))
     # half the rows with raw random scale fields, half with the scales
     # pinned near 1 (the selftest's choice) so that no row overflows
     w = np.concatenate([raw[:nbytes // 2], mg.sane_scales(t, raw[nbytes // 2:])]).reshape(n, -1)
     want = oracle.f16_bits_to_f32(oracle.dequant(t, w.reshape(-1), n * k)).reshape(n, k)
     ok = np.isfinite(want).all(axis=1)
     x = np.eye(k, dtype=np.float32)
-    hip.set_gemm_tile(bn)
+    if isinstance(bn, int):
+        hip.set_gemm_tile(bn)
+    else:
+        hip.set_gemm_plan(256, 256)
     try:
         y, _ = run(hip, t, w, x, k, n, k, gguf.DT_F16, gguf.DT_F32)
     finally:
         hip.set_gemm_tile(0)
+        hip.set_gemm_plan(0, 0)
     got = y.T  # [n, k]
     assert np.array_equal(got[ok], want[ok]), (int(ok.sum()), np.argwhere(got[ok] != want[ok])[:4])
 
@@ -173,8 +177,10 @@ def test_gemm_narrow_weight_many_tokens(hip, n, k, m):
     assert rel(y, want) <= 1e-5
 
 
-@pytest.mark.parametrize("m", [16, 64, 256], ids=["sk16", "reg_a", "lds_pipe"])
-def test_gemm_x_range_flags(hip, m):
+@pytest.mark.parametrize("plan", [(16, 16), (32, 16), (64, 32), (64, 64), (64, 128), (128, 256), (256, 256)],
+                         ids=lambda p: f"{p[0]}x{p[1]}")
+@pytest.mark.parametrize("m", [16, 64, 256])
+def test_gemm_x_range_flags(hip, m, plan):
     """bf16 X beyond f16's range, or too small for it, no longer turns into
     inf / zero silently: the tiles flag it (cima_hip_gemm_status) on every
     tile kind, for the GGUF and the bitsandbytes weights; in-range bf16 and
@@ -183,7 +189,14 @@ def test_gemm_x_range_flags(hip, m):
     w = torch.from_numpy(synth.weights(Q4_K, 70, 0.02, n, k)).cuda()
     y = torch.empty((m, n), device="cuda")
     hip.gemm_status(clear=True)
+    hip.set_gemm_plan(*plan)
+    try:
+        _check_x_range_flags(hip, m, n, k, w, y)
+    finally:
+        hip.set_gemm_plan(0, 0)
 
+
+def _check_x_range_flags(hip, m, n, k, w, y):
     def flags(x, xd):
         hip.gguf_gemm(Q4_K, x, w, y, m, n, k, n, xd, gguf.DT_F32)
         return hip.gemm_status(clear=True)
