@@ -163,6 +163,13 @@ const char* const kModuleFiles[NUM_MODULES] = {"cima_gemv_a.hsaco", "cima_gemv_b
                                                "cima_gemm.hsaco",   "cima_dequant.hsaco", "cima_decode.hsaco",
                                                "cima_bnb4.hsaco",   "cima_gemm_wide.hsaco"};
 
+// weights and X types with _b16l_ kernels, the 32 x 16 prefill tiles for grids
+// of at most one workgroup per CU (sk16_serial in gguf_gemm.hip)
+bool gemm_b16l(const char* weights, const char* xt) {
+    return !strcmp(weights, "q4_k") || !strcmp(weights, "q5_k") || !strcmp(weights, "iq4_xs") ||
+           (!strcmp(weights, "nf4") && !strcmp(xt, "f16"));
+}
+
 // decode-step kernels (cima_decode.hsaco)
 const char* const kDecodeKernels[] = {
     "cima_rmsnorm_f16",     "cima_rope_f16",        "cima_kv_append_f16",    "cima_attn_split_d64",
@@ -579,6 +586,13 @@ int cima_hip_init(int device, const char* code_dir, cima_hip_ctx** out) {
                         if (!rc) rc = add(MOD_GEMM, name);
                     }
                 }
+    for (const char* wn : {"q4_k", "q5_k", "iq4_xs", "nf4"})
+        for (const char* xt : {"f32", "f16", "bf16"})
+            for (const char* yt : {"f32", "f16"}) {
+                char name[96];
+                snprintf(name, sizeof name, "cima_gemm_%s_b16l_%s_%s", wn, xt, yt);
+                if (!rc && gemm_b16l(wn, xt)) rc = add(MOD_GEMM, name);
+            }
     for (const char* wn : {"q8_0", "q4_0", "q4_1", "q5_0", "q5_1", "q4_k", "q5_k", "q6_k", "iq4_xs", "nf4", "f16w"})
         for (const char* xt : {"f16", "bf16"})
             for (const char* yt : {"f32", "f16"}) {
@@ -969,8 +983,10 @@ int gemm_launch(cima_hip_ctx* ctx, const char* fname, const void* x, const void*
     static const char* const kn[] = {"b16", "b16n", "b32", "b64", "b128", "b256", "w256"};
     // a split group tile writes fp32 partial tiles through its Y
     const bool part_y = ks > 1 && !sk;
+    const unsigned gx = (unsigned)((n + bm - 1) / bm), gy = (unsigned)((m + bn - 1) / bn);
+    const bool low = p.kind == KB16 && (long long)gx * gy * ks <= ctx->num_cu && gemm_b16l(fname, xn[x_dtype]);
     char name[96];
-    snprintf(name, sizeof name, "cima_gemm_%s_%s_%s_%s", fname, kn[p.kind], xn[x_dtype],
+    snprintf(name, sizeof name, "cima_gemm_%s_%s_%s_%s", fname, low ? "b16l" : kn[p.kind], xn[x_dtype],
              y_dtype == CIMA_DT_F32 || part_y ? "f32" : "f16");
     hipFunction_t f;
     if (int rc = get_fn(ctx, name, &f)) return rc;
@@ -980,7 +996,6 @@ int gemm_launch(cima_hip_ctx* ctx, const char* fname, const void* x, const void*
     int mm = m, nn = n, kk = k, ld = part_y ? n : ldy;
     GemmExt ge = gext;
     ge.status = ctx->gemm_xcheck ? ctx->gemm_status : nullptr;
-    const unsigned gx = (unsigned)((n + bm - 1) / bm), gy = (unsigned)((m + bn - 1) / bn);
     ge.part = ks > 1 ? part : nullptr;
     ge.ksplit = ks;
     void* args[] = {&xa, &wa, &ya, &mm, &nn, &kk, &ld, &ge};

@@ -486,6 +486,70 @@ DEV void deq(const typename D::Ctx& c, const typename D::Raw& r, const uint8_t* 
     for (int i = 0; i < 8; i++) D::part(c, r, p, j, i, o[2 * i], o[2 * i + 1]);
 }
 
+// The whole sub-block by byte conversions (v_cvt_f32_ubyte) and f2h2, whose
+// operands the compiler does not see through: more instructions than part(),
+// the same bits.  The 16-token tiles wait on memory rather than on
+// instruction issue, and for these formats some of them are faster this way
+// (sk16_serial in gguf_gemm.hip).
+template <typename D>
+struct SerialDeq;
+template <>
+struct SerialDeq<GG<DQ4_K>> {
+    DEV static void deq(const GG<DQ4_K>::Ctx&, const DQ4_K::Raw& r, int j, uint32_t (&o)[16]) {
+        uint32_t sc0, m0, sc1, m1;
+        q4k_scales(r.h, (j & 7) >> 1, sc0, m0, sc1, m1);
+        const bool hi = j & 1;
+        const float ds = h2f(r.h.x & 0xffffu) * (float)(hi ? sc1 : sc0), mm = h2f(r.h.x >> 16) * (float)(hi ? m1 : m0);
+        const uint32_t q[8] = {r.q0.x, r.q0.y, r.q0.z, r.q0.w, r.q1.x, r.q1.y, r.q1.z, r.q1.w};
+        const int sh = hi ? 4 : 0;
+#pragma unroll
+        for (int i = 0; i < 8; i++) bytes_affine((q[i] >> sh) & 0x0F0F0F0Fu, ds, -mm, o[2 * i], o[2 * i + 1]);
+    }
+};
+template <>
+struct SerialDeq<GG<DQ5_K>> {
+    DEV static void deq(const GG<DQ5_K>::Ctx&, const DQ5_K::Raw& r, int j, uint32_t (&o)[16]) {
+        const int s = j & 7;
+        uint32_t sc0, m0, sc1, m1;
+        q4k_scales(r.h, s >> 1, sc0, m0, sc1, m1);
+        const bool hi = s & 1;
+        const float ds = h2f(r.h.x & 0xffffu) * (float)(hi ? sc1 : sc0), mm = h2f(r.h.x >> 16) * (float)(hi ? m1 : m0);
+        const uint32_t q[8] = {r.q0.x, r.q0.y, r.q0.z, r.q0.w, r.q1.x, r.q1.y, r.q1.z, r.q1.w};
+        const uint32_t h[8] = {r.qh0.x, r.qh0.y, r.qh0.z, r.qh0.w, r.qh1.x, r.qh1.y, r.qh1.z, r.qh1.w};
+        const int sh = hi ? 4 : 0;
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            bytes_affine(((q[i] >> sh) & 0x0F0F0F0Fu) | (((h[i] >> s) & 0x01010101u) << 4), ds, -mm, o[2 * i],
+                         o[2 * i + 1]);
+    }
+};
+template <>
+struct SerialDeq<GG<DIQ4_XS>> {
+    DEV static void deq(const GG<DIQ4_XS>::Ctx&, const DIQ4_XS::Raw& r, int j, uint32_t (&o)[16]) {
+        const float dl = iq4xs_dl(r.hdr, j & 7);
+        const uint32_t q[4] = {r.q.x, r.q.y, r.q.z, r.q.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            bytes_affine(iq4nl_bytes(q[i] & 0x0F0F0F0Fu) ^ 0x80808080u, dl, -128.f * dl, o[2 * i], o[2 * i + 1]);
+            bytes_affine(iq4nl_bytes((q[i] >> 4) & 0x0F0F0F0Fu) ^ 0x80808080u, dl, -128.f * dl, o[8 + 2 * i],
+                         o[8 + 2 * i + 1]);
+        }
+    }
+};
+template <>
+struct SerialDeq<DNF4> {
+    DEV static void deq(const DNF4::Ctx& c, const DNF4::Raw& r, int, uint32_t (&o)[16]) {
+        const uint32_t w[4] = {r.q.x, r.q.y, r.q.z, r.q.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                const uint32_t byte = (w[i] >> (8 * b)) & 0xFFu;
+                o[4 * i + b] = f2h2(c.code[byte >> 4] * r.a, c.code[byte & 0xFu] * r.a);
+            }
+    }
+};
+
 // D::init with the codebook for DNF4, nothing for the others
 template <typename D>
 DEV void fmt_init(const typename D::Ctx& c, const GemmExt& e) {

@@ -21,7 +21,12 @@
 // +8) of token l % 16, read from the split's activation tile in LDS (the
 // split's RT waves stage it together).  The four splits' partial tiles are
 // summed through LDS at the end.
-template <typename D, int XT, int YT, int PF, int RT>
+//
+// Bound by memory round trips, with one or two stages in flight per wave, so
+// the order of a stage's instructions counts.  SER: weights and X by
+// SerialDeq and f2h2.  EARLY: the loads of the stage after next go out
+// before the barrier of this one.
+template <typename D, int XT, int YT, int PF, int RT, bool SER, bool EARLY>
 __device__ void gemm_body_sk16(const void* __restrict__ x, const uint8_t* __restrict__ w, void* __restrict__ y,
                                int m, int n, int k, int ldy, const GemmExt& ext) {
     constexpr int ES = XT == XT_F32 ? 4 : 2, KP = 136;  // tile pitch in halves (pads away bank conflicts)
@@ -61,16 +66,17 @@ __device__ void gemm_body_sk16(const void* __restrict__ x, const uint8_t* __rest
     for (int i = 0; i < PF; i++) issue(ring[i], i);
     auto step = [&](Stage& st, int i, bool next) {
         const int buf = i & 1;
+        auto xcvt = [](float lo, float hi) { return SER ? f2h2(lo, hi) : pack_f16(lo, hi); };
         // the lane's activations -> f16 in the split's tile
         uint4* dst = reinterpret_cast<uint4*>(&xl[buf][ks][xtok * KP + xk]);
         if constexpr (XT == XT_F32) {
 #pragma unroll
             for (int j = 0; j < XW / 2; j++) {
                 const uint4 a = st.xr[2 * j], b = st.xr[2 * j + 1];
-                dst[j] = make_uint4(pack_f16(__builtin_bit_cast(float, a.x), __builtin_bit_cast(float, a.y)),
-                                    pack_f16(__builtin_bit_cast(float, a.z), __builtin_bit_cast(float, a.w)),
-                                    pack_f16(__builtin_bit_cast(float, b.x), __builtin_bit_cast(float, b.y)),
-                                    pack_f16(__builtin_bit_cast(float, b.z), __builtin_bit_cast(float, b.w)));
+                dst[j] = make_uint4(xcvt(__builtin_bit_cast(float, a.x), __builtin_bit_cast(float, a.y)),
+                                    xcvt(__builtin_bit_cast(float, a.z), __builtin_bit_cast(float, a.w)),
+                                    xcvt(__builtin_bit_cast(float, b.x), __builtin_bit_cast(float, b.y)),
+                                    xcvt(__builtin_bit_cast(float, b.z), __builtin_bit_cast(float, b.w)));
             }
         } else {
 #pragma unroll
@@ -80,17 +86,26 @@ __device__ void gemm_body_sk16(const void* __restrict__ x, const uint8_t* __rest
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     o[e] = XT == XT_F16 ? v[e]
-                                        : pack_f16(__builtin_bit_cast(float, v[e] << 16),
+                                        : xcvt(__builtin_bit_cast(float, v[e] << 16),
                                                __builtin_bit_cast(float, v[e] & 0xffff0000u));
                 }
                 dst[j] = make_uint4(o[0], o[1], o[2], o[3]);
             }
         }
         uint32_t o[16];
-        deq<D>(dc, st.wr, wp, 4 * (s0 + min(ks + 4 * i, nk - 1)) + g, o);
-        __syncthreads();
-        if (next) issue(st, i + PF);
-        __builtin_amdgcn_sched_barrier(0);
+        const int jw = 4 * (s0 + min(ks + 4 * i, nk - 1)) + g;
+        if constexpr (SER) SerialDeq<D>::deq(dc, st.wr, jw, o);
+        else deq<D>(dc, st.wr, wp, jw, o);
+        if constexpr (EARLY) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (next) issue(st, i + PF);
+            __builtin_amdgcn_sched_barrier(0);
+            __syncthreads();
+        } else {
+            __syncthreads();
+            if (next) issue(st, i + PF);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         if (ks + 4 * i < nk) {
 #pragma unroll
             for (int q = 0; q < 4; q++) {
@@ -154,6 +169,20 @@ constexpr int group_occ() { return BN == 32 && XT != XT_F32 && sizeof(typename D
 template <int BN, int XT>
 constexpr int group_rg() { return BN == 128 && XT == XT_F32 ? 4 : 2; }
 
+// 32-row 16-token tiles with SerialDeq where several workgroups share a CU
+// (measured on MI355X, cold, us, part() / SerialDeq: Q4_K, bf16 X, 14336x4096
+// at 16 tokens 17.7 / 17.3, 28672x4096 35.8 / 32.6; Q5_K 28.2 / 25.7 and 52.8 /
+// 48.4; IQ4_XS 17.5 / 16.6; NF4, f16 X, 28672x4096 32.2 / 30.0); the other
+// formats are no faster that way (Q4_1 16.1 / 16.2, Q5_1 16.3 / 18.1, NF4,
+// bf16 X, 16.3 / 21.9), and nor is a grid of at most one workgroup per CU,
+// which for these formats has kernels of its own, _b16l_ (8192x4096: Q4_K
+// 12.7 / 12.9, IQ4_XS 11.2 / 12.5, Q5_K 17.7 / 18.7).
+template <typename D, int XT>
+constexpr bool sk16_serial() {
+    return std::is_same<D, GG<DQ4_K>>::value || std::is_same<D, GG<DQ5_K>>::value ||
+           std::is_same<D, GG<DIQ4_XS>>::value || (std::is_same<D, DNF4>::value && XT == XT_F16);
+}
+
 // name: cima_gemm_<fmt>_b<BN>_<x type>_<y type>
 // (HIP's second bound is the minimum waves per SIMD: the 16-token tiles
 // ask for 4, two 512-thread workgroups per CU, which the compiler then
@@ -163,7 +192,8 @@ constexpr int group_rg() { return BN == 128 && XT == XT_F32 ? 4 : 2; }
     extern "C" __global__ __launch_bounds__(512, (BN == 16 ? 4 : BN == 256 ? 2 : group_occ<D, BN, XT>())) void \
     cima_gemm_##FN##_b##BN##_##XN##_##YN(                                                             \
         const void* x, const uint8_t* w, void* y, int m, int n, int k, int ldy, GemmExt ext) {      \
-        if constexpr (BN == 16) gemm_body_sk16<D, XT, YT, 1, 2>(x, w, y, m, n, k, ldy, ext);         \
+        if constexpr (BN == 16)                                                                       \
+            gemm_body_sk16<D, XT, YT, 1, 2, sk16_serial<D, XT>(), false>(x, w, y, m, n, k, ldy, ext); \
         else if constexpr (BN == 256) gemm_wide<D, XT, YT, 2, 2, 2, 4>(x, w, y, m, n, k, ldy, ext);   \
         else \
             gemm_group<D, XT, YT, BN / 32, group_rg<BN, XT>(), 8 / group_rg<BN, XT>(), group_pf<D, BN>()>(x, w, y, m, n, k, ldy, ext); \
@@ -189,11 +219,19 @@ constexpr int sk16n_pf() {
                ? 2
                : 1;
 }
+//
+// Their next loads go out before the barrier, with the spread decoders
+// (measured on MI355X, 16 tokens, us, SerialDeq and loads behind the barrier /
+// part() and loads behind / part() and loads before: Q4_K, f16 X, 4096x14336
+// 23.9 / 25.1 / 23.1, 4096x4096 8.5 / 8.0 / 7.9; bf16 X 25.7 / 27.9 / 25.8
+// and 9.4 / 9.5 / 9.0), but for NF4, whose table lookups are faster in one
+// go (f16 X, 4096x14336 21.4 / 27.0 / 27.4, 4096x4096 7.8 / 8.9 / 9.1).
 #define GEMM_KERNEL_NARROW(FN, D, XT, XN, YT, YN)                                                   \
     extern "C" __global__ __launch_bounds__(256, (sk16n_pf<D, XT>() == 2 ? 3 : 4)) void            \
     cima_gemm_##FN##_b16n_##XN##_##YN(const void* x, const uint8_t* w, void* y, int m, int n, int k, \
                                       int ldy, GemmExt ext) {                                       \
-        gemm_body_sk16<D, XT, YT, sk16n_pf<D, XT>(), 1>(x, w, y, m, n, k, ldy, ext);                \
+        constexpr bool nf4 = std::is_same<D, DNF4>::value;                                          \
+        gemm_body_sk16<D, XT, YT, sk16n_pf<D, XT>(), 1, nf4, !nf4>(x, w, y, m, n, k, ldy, ext);     \
     }
 #define GEMM_XY_NARROW(FN, D)                                                 \
     GEMM_KERNEL_NARROW(FN, D, XT_F32, f32, XT_F32, f32)                       \
@@ -202,6 +240,14 @@ constexpr int sk16n_pf() {
     GEMM_KERNEL_NARROW(FN, D, XT_F32, f32, XT_F16, f16)                       \
     GEMM_KERNEL_NARROW(FN, D, XT_F16, f16, XT_F16, f16)                       \
     GEMM_KERNEL_NARROW(FN, D, XT_BF16, bf16, XT_F16, f16)
+#define GEMM_KERNEL_LOW(FN, D, XT, XN, YT, YN)                                                      \
+    extern "C" __global__ __launch_bounds__(512, 4) void cima_gemm_##FN##_b16l_##XN##_##YN(         \
+        const void* x, const uint8_t* w, void* y, int m, int n, int k, int ldy, GemmExt ext) {      \
+        static_assert(sk16_serial<D, XT>(), "_b16_ is the same kernel");                            \
+        gemm_body_sk16<D, XT, YT, 1, 2, false, false>(x, w, y, m, n, k, ldy, ext);                  \
+    }
+#define GEMM_XY_LOW(FN, D, XT, XN) GEMM_KERNEL_LOW(FN, D, XT, XN, XT_F32, f32) GEMM_KERNEL_LOW(FN, D, XT, XN, XT_F16, f16)
+#define GEMM_LOW(FN, D) GEMM_XY_LOW(FN, D, XT_F32, f32) GEMM_XY_LOW(FN, D, XT_F16, f16) GEMM_XY_LOW(FN, D, XT_BF16, bf16)
 #define GEMM_FMT(FN, D) \
     GEMM_XY(FN, D, 16) GEMM_XY_NARROW(FN, D) GEMM_XY(FN, D, 32) GEMM_XY(FN, D, 64) GEMM_XY(FN, D, 128) GEMM_XY(FN, D, 256)
 
@@ -217,6 +263,10 @@ GEMM_FMT(iq4_xs, GG<DIQ4_XS>)
 // bitsandbytes 4-bit weights decoded in the tiles, and plain f16 weights
 GEMM_FMT(nf4, DNF4)
 GEMM_FMT(f16w, DF16)
+GEMM_LOW(q4_k, GG<DQ4_K>)
+GEMM_LOW(q5_k, GG<DQ5_K>)
+GEMM_LOW(iq4_xs, GG<DIQ4_XS>)
+GEMM_XY_LOW(nf4, DNF4, XT_F16, f16)
 
 // f16 weights of any k (the slab route for k % 64 != 0): one thread per
 // output, X rounded to f16 as the tiles round it, fp32 accumulation in k

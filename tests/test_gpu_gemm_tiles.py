@@ -211,3 +211,39 @@ def test_planned_k_split_of_the_wide_group_tiles(hip, t, m, n, k, xd, plan):
     want = x.float().cpu().numpy().astype(np.float16).astype(np.float64) @ w16.reshape(256, k).astype(np.float64).T
     assert rel(y.cpu().numpy()[:, rows], want) <= 1e-5
     assert bool((slab != 0).any())
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, IQ4_XS, 0], ids=["q4_k", "q5_k", "iq4_xs", "nf4"])
+@pytest.mark.parametrize("k", [256, 768, 1280])
+def test_32_row_tiles_of_full_and_low_grids(hip, t, k):
+    """The 16-token tiles decode in one way where several workgroups share a
+    CU (257 row tiles here) and in another below (slices of 4096 rows, at
+    most 128 tiles): the same bits, at 2, 6 and 10 stages."""
+    n, m, bs = 8225, 13, 64
+    rng = np.random.default_rng(k)
+    if t:
+        w = torch.from_numpy(synth.weights(t, 300 + t, 0.02, n, k).reshape(n, -1)).cuda()
+    else:
+        w = torch.from_numpy(rng.integers(0, 256, (n, k // 2), dtype=np.uint8)).cuda()
+        absmax = torch.from_numpy((rng.random((n, k // bs)) + 0.01).astype(np.float32)).cuda()
+        qmap = torch.from_numpy(nf4.NF4_CODE.copy()).cuda()
+        slab = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
+
+    def mul(x, r0, r1, yd):
+        y = torch.full((m, r1 - r0), float("nan"), dtype=TDT[yd], device="cuda")
+        if t:
+            hip.gguf_gemm(t, x, w[r0:r1], y, m, r1 - r0, k)
+        else:
+            hip.nf4_gemm_slab(x, w[r0:r1], absmax[r0:r1], qmap, y, m, r1 - r0, k, bs, slab)
+        return y
+
+    hip.set_gemm_plan(32, 16)
+    try:
+        for xd, yd in ((BF16, F32), (F16, F16), (F32, F32)):
+            x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(TDT[xd]).cuda()
+            whole = mul(x, 0, n, yd)
+            parts = torch.cat([mul(x, r, min(r + 4096, n), yd) for r in range(0, n, 4096)], 1)
+            torch.cuda.synchronize()
+            assert torch.equal(whole, parts) and bool(torch.isfinite(whole).all()), (xd, yd)
+    finally:
+        hip.set_gemm_plan(0, 0)
