@@ -4,7 +4,8 @@ transformer.rs:618-655) decodes W into an f16 slab with gguf_dequant and
 multiplies it with cublasGemmEx (src/cuda.rs:2468-2541); here the same
 call runs the fused MFMA kernels, which dequantise W bit-exactly tile by
 tile, so W is never expanded and no library GEMM runs; the slab only holds
-the partial tiles of narrow weights split along k at up to 32 tokens.  Checked
+the partial tiles of narrow weights split along k (at tiles of up to 128
+tokens).  Checked
 against the CPU path (f16 dequant + fp64 GEMM of the f16-rounded X): 1e-5
 with fp32 Y, where only the summation order differs, and the north star's
 1e-3 with f16 Y."""
@@ -13,7 +14,7 @@ import pytest
 
 import oracle
 from cima_amd import gguf, synth
-from cima_amd.hip import EngineError, E_INVALID
+from cima_amd.hip import EngineError, E_INVALID, gemm_plan
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -139,11 +140,22 @@ def test_slab_entry_k_split(hip, t, n, k, m):
     against the CPU path (1e-5), against the unsplit product (1e-6: only
     the order of the k sum differs), bit-identical run to run and in a
     replayed graph; a slab too small for the partials runs unsplit, giving
-    cima_hip_gguf_gemm's bits."""
+    cima_hip_gguf_gemm's bits.  Shapes that are planned unsplit are forced
+    to split in two on their planned tile."""
+    rows, tokens, ks = gemm_plan(t, m, n, k, gguf.DT_BF16, 32 << 20, hip.num_cu)
+    if ks == 1:
+        hip.set_gemm_plan(rows, tokens, 2)
+    try:
+        _check_k_split(hip, t, n, k, m, max(ks, 2))
+    finally:
+        hip.set_gemm_plan(0, 0, 0)
+
+
+def _check_k_split(hip, t, n, k, m, ks):
     w = synth.weights(t, 130, 0.02, n, k)
     wd = torch.from_numpy(w).cuda()
     x = torch.from_numpy(synth.normal(131 + m, 1.0, m * k).reshape(m, k)).to(torch.bfloat16).cuda()
-    slab = torch.empty(32 << 20, dtype=torch.uint8, device="cuda")
+    slab = torch.full((32 << 20,), 0x5A, dtype=torch.uint8, device="cuda")
     y1 = torch.empty((m, n), device="cuda")
     y2 = torch.empty((m, n), device="cuda")
     yu = torch.empty((m, n), device="cuda")
@@ -152,6 +164,9 @@ def test_slab_entry_k_split(hip, t, n, k, m):
     hip.gguf_gemm(t, x, wd, yu, m, n, k)
     torch.cuda.synchronize()
     assert torch.equal(y1, y2)
+    # every partial tile is in the slab, nothing past them
+    assert all(bool((p != 0x5A).any()) for p in slab[:4 * ks * m * n].view(ks, -1))
+    assert bool((slab[4 * ks * m * n:] == 0x5A).all())
     got, unsplit = y1.cpu().numpy(), yu.cpu().numpy()
     assert rel(got, unsplit) <= 1e-6
     w16 = oracle.f16_bits_to_f32(oracle.dequant(t, w, n * k)).reshape(n, k)
