@@ -1358,7 +1358,12 @@ int cima_hip_decode_step(cima_hip_ctx* ctx, const cima_decoder* d) {
     // The split partials are merged by a launch of their own (into the q
     // part of qkv, which the attention launch has consumed) rather than in
     // every workgroup of the o projection where the partials of a full cache
-    // pass 128 KB: each of the projection's workgroups reads all live ones.
+    // pass 128 KB.  Inside, each of the projection's workgroups reads, per
+    // head, up to 32 (m, l) pairs and 16 partial rows whatever the position
+    // (their loads go out before it is known), and every further live chunk:
+    // a cost of the cache's capacity first, of the position then.  The rule
+    // cannot look at the position, which a replayed graph reads on the
+    // device; its line is the one between two measured sizes, 118 and 133 KB.
     // Measured on MI355X, us per step, merged inside / apart: Llama-3-8B
     // layers (4 of them, Q4_K) at position 10 of 1024 (133 KB) 217 / 194, 1000
     // of 2048 226 / 198, 10 of 8192 245 / 211, 8000 of 8192 373 / 220;

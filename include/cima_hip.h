@@ -379,7 +379,9 @@ typedef struct cima_decoder {
     const cima_decoder_layer* layers;  /* host array of n_layers */
     /* workspace, all device memory */
     void* x;          /* f16 [hidden] residual stream */
-    void* qkv;        /* f16 [(q_heads + 2 kv_heads) * head_dim] */
+    void* qkv;        /* f16 [(q_heads + 2 kv_heads) * head_dim]; scratch: a step whose
+                       * partials are merged in a launch of their own leaves the
+                       * merged attention in the q part */
     void* act;        /* f16 [ffn] */
     void* logits;     /* f16 [vocab] */
     float* part;      /* q_heads * ceil(max_seq / attn_chunk) * (head_dim + 2) floats */
@@ -396,7 +398,10 @@ typedef struct cima_decoder {
  * pos += 1.  Replaces
  * enqueue_decode_device (src/models/transformer.rs:1440-1461) and
  * forward_chunk_at's rows == 1 path (:1012-1300): 5 launches per layer
- * where the reference issues about 12 (7 with separate q, k, v matrices). */
+ * where the reference issues about 12 (7 with separate q, k, v matrices).
+ * Where the partials of a full cache, q_heads * ceil(max_seq / attn_chunk) *
+ * (head_dim + 2) floats, pass 128 KB, the merge is a launch of its own: 6
+ * per layer (8 with separate matrices). */
 int cima_hip_decode_step(cima_hip_ctx* ctx, const cima_decoder* d);
 
 /* ---------------------------------------------------------------------
