@@ -865,37 +865,73 @@ int plan_bn(GemmKind kind) {
     return bn[kind];
 }
 
+// workgroups of a plan
+double plan_wgs(GemmPlan p, int m, int n, int x_dtype) {
+    const int bm = plan_bm(p.kind, x_dtype), bn = plan_bn(p.kind);
+    return (double)((n + bm - 1) / bm) * ((m + bn - 1) / bn) * p.ksplit;
+}
+
 // Estimated time (us) of a plan on MI355X: rounds of workgroups over the
 // CUs, each a fixed cost (first loads, staging, output) plus its k stages.
 // The constants are fits to cold runs (Q4_K, bf16 X) of one round at k =
-// 4096 and 14336 -- us per 64-k stage and fixed us: b32 0.20 / 5, b64 0.215
-// / 9.5, b128 0.27 / 13.5, b256 0.81 / 20, w256 1.5 / 20 -- and of the
-// 16-token tiles per 512-k step: 1.5 with one workgroup per CU, 2.05 with
-// two (b16), 0.95 and 1.6 (b16n); `heavy` formats (Q5_K, Q6_K) decode at
-// about 1.7 times that.  A second resident workgroup does not speed the
+// 4096 and 14336, the fixed cost the part that does not grow with k -- us
+// per 64-k stage and fixed us: b32 0.20 / 5, b64 0.215 / 9.5, b128 0.27 /
+// 13.5, b256 0.81 / 20, w256 1.5 / 20; heavy formats (Q5_K, Q6_K) decode
+// at about 1.7 times that.  A second resident workgroup does not speed the
 // 64-row tiles up (b32 at 14336 rows: 224 workgroups 17.8, 448 34).  The
 // k-split adds the partial tiles' traffic and the summing launch.  Estimated
-// against measured at 14336x4096: 16 / 32 / 64 / 128 / 512 / 2048 tokens 17
-// / 18 / 23 / 31 / 72 / 232 against 17 / 18 / 23 / 31 / 76 / 260; split
-// against unsplit, measured: 4096x14336 at 16 / 100 tokens 19 / 25 and 39 /
-// 111 (Q6_K), 6144x4096 at 32 13.6 / 17, 1024x4096 at 16 9.8 / 9.0 (Q4_K, not
-// split) and 10.9 / 12.3 (Q6_K, split).
-double plan_cost(int cu, GemmPlan p, int m, int n, int k, int x_dtype, bool heavy) {
-    const int bm = plan_bm(p.kind, x_dtype), bn = plan_bn(p.kind);
-    const double wgs = (double)((n + bm - 1) / bm) * ((m + bn - 1) / bn) * p.ksplit;
+// against measured at 14336x4096: 64 / 128 / 512 / 2048 tokens 23 / 31 / 72
+// / 232 against 23 / 31 / 73 / 260; split against unsplit, measured:
+// 4096x14336 at 100 tokens 39 / 111 (Q6_K).
+double plan_cost(int cu, GemmPlan p, int m, int n, int k, int x_dtype, const char* fname) {
+    static const double stage[] = {0, 0, 0.20, 0.215, 0.27, 0.81, 1.5}, fixed[] = {0, 0, 5, 9.5, 13.5, 20, 20};
+    const bool heavy = !strcmp(fname, "q5_k") || !strcmp(fname, "q6_k");
+    const double wide_f32 = p.kind == KB128 && x_dtype == CIMA_DT_F32 ? 2.0 : 1.0;
+    const double rounds = (double)(((long long)plan_wgs(p, m, n, x_dtype) + cu - 1) / cu);
+    double t = rounds * (k / 64 / (double)p.ksplit * stage[p.kind] * wide_f32 * (heavy ? 1.7 : 1.0) + fixed[p.kind]);
+    if (p.ksplit > 1) t += 3.5 + ((double)p.ksplit * 8 + 4) * m * n / 3e6;
+    return t;
+}
+
+// Decoding in short_cost against Q4_K's: b16n at one workgroup per CU and
+// beyond, b16 likewise, b32 (null: f16 weights, as Q4_K)
+const double* short_decode(const char* fname) {
+    struct Decode { const char* fmt; double f[5]; };
+    static const Decode decode[] = {
+        {"q4_k", {1, 1, 1, 1, 1}},                     {"q8_0", {1.02, 1.09, 1.12, 1.11, 1.22}},
+        {"q6_k", {1.54, 1.34, 1.59, 1.78, 2.03}},      {"q5_k", {1.24, 1.18, 1.31, 1.48, 1.52}},
+        {"iq4_xs", {0.97, 0.88, 0.84, 0.86, 0.86}},    {"q4_0", {0.89, 0.88, 0.89, 0.79, 0.80}},
+        {"q4_1", {0.91, 0.91, 0.91, 0.83, 0.85}},      {"q5_0", {0.92, 0.90, 0.90, 0.82, 0.85}},
+        {"q5_1", {0.93, 0.92, 0.93, 0.86, 0.88}},      {"nf4", {1.09, 0.95, 1.08, 0.91, 0.93}}};
+    for (const Decode& d : decode)
+        if (!strcmp(d.fmt, fname)) return d.f;
+    return nullptr;
+}
+
+// The same for up to 32 tokens: b16n and b16, a fixed cost plus 512-k steps
+// whose cost depends on the workgroups per CU, and b32 as above, each with a
+// factor for the format's decoding and one for the X type.  Fits to every
+// plan of 19 weights (512 to 28672 rows, k 896 to 14336), ten formats, three
+// X types, 16 and 32 tokens, cold (9 to 10 % rms).
+double short_cost(int cu, GemmPlan p, int m, int n, int k, int x_dtype, const double* decode) {
+    const double wgs = plan_wgs(p, m, n, x_dtype), per_cu = (double)(((long long)wgs + cu - 1) / cu);
+    const int tile = p.kind == KB16N ? 0 : p.kind == KB16 ? 1 : 2, c = tile == 2 ? 4 : 2 * tile + (per_cu > 1);
+    static const double f32x[5] = {1.95, 2.02, 1.33, 1.54, 1.23}, bf16x[5] = {1.18, 1.07, 1.11, 1.10, 1.06};
+    double f = x_dtype == CIMA_DT_F32 ? f32x[c] : x_dtype == CIMA_DT_BF16 ? bf16x[c] : 1.0;
+    if (decode) f *= decode[c];
     double t;
-    if (p.kind == KB16 || p.kind == KB16N) {
-        const bool n16 = p.kind == KB16N;
-        const double steps = (k + 511) / 512 / (double)p.ksplit;
-        const double two = (n16 ? 1.6 : 2.05) * (wgs > 2 * cu ? wgs / (2 * cu) : 1.0);
-        t = 1.0 + steps * (heavy ? 1.7 : 1.0) * (wgs <= cu ? (n16 ? 0.95 : 1.5) : two);
+    if (tile == 2) {
+        t = per_cu * (k / 64.0 / p.ksplit * 0.217 * f + 3.5);
     } else {
-        static const double stage[] = {0, 0, 0.20, 0.215, 0.27, 0.81, 1.5}, fixed[] = {0, 0, 5, 9.5, 13.5, 20, 20};
-        const double wide_f32 = p.kind == KB128 && x_dtype == CIMA_DT_F32 ? 2.0 : 1.0;
-        const double rounds = (double)(((long long)wgs + cu - 1) / cu);
-        t = rounds * (k / 64 / (double)p.ksplit * stage[p.kind] * wide_f32 * (heavy ? 1.7 : 1.0) + fixed[p.kind]);
+        static const double fixed[] = {3.05, 2.65}, one[] = {0.67, 1.17}, two[] = {1.32, 1.82}, more[] = {0.69, 0.94};
+        t = fixed[tile] +
+            k / 512.0 / p.ksplit * f * (per_cu <= 1 ? one[tile] : per_cu <= 2 ? two[tile] : more[tile] * per_cu);
     }
-    if (p.ksplit > 1) t += (p.kind <= KB16N ? 6.0 : 3.5) + ((double)p.ksplit * 8 + 4) * m * n / 3e6;
+    // partial tiles and the summing launch (fewer than 16 tokens cost no
+    // less: 6144x4096 Q4_K, bf16 X, at 2 tokens 13.2 in two ranges, 15.9 in
+    // four)
+    static const double sum[] = {1.8, 2.2, 3.0}, rate[] = {0.78e6, 1.12e6, 3.64e6};
+    if (p.ksplit > 1) t += sum[tile] + ((double)p.ksplit * 8 + 4) * ((m + 15) / 16 * 16) * n / rate[tile];
     return t;
 }
 
@@ -907,31 +943,49 @@ struct GemmTune {
     int ksplit = 0;  // 0 = planned, 1 = none, else this many where they divide and fit
 };
 
-// The cheapest plan by plan_cost: 16-token tiles up to 32 tokens, every
+// The cheapest plan by its estimate: 16-token tiles up to 32 tokens, every
 // wider tile that is at most twice the tokens (a wider one only pads), k
 // split 2 or 4 ways where the slab holds the partial tiles (S x m x n fp32),
 // the stages divide evenly and every split keeps at least eight 64-k
 // stages (four 128-k stages, one per wave, for the 16-token tiles).
-GemmPlan plan_gemm(const GemmTune& tune, int num_cu, int m, int n, int k, int x_dtype, bool heavy, size_t part_bytes) {
+//
+// Up to 32 tokens the estimates lie closer together than they are exact, so
+// a 16-token plan by the CUs' fill stands unless the cheapest is estimated 12 %
+// below it: 16-row tiles where 32-row ones would fill at most half the CUs,
+// split four ways at a quarter workgroup per CU and two ways at a half;
+// 32-row ones split two ways at one; no split up to 2048 k, where the summing
+// launch costs more than it saves (Q4_K, bf16 X, 16 tokens: 512x2048 6.06
+// whole / 6.60 in four, 2048x2048 6.33 / 7.30 in two, but 1024x4096 9.05 /
+// 7.92 in four).  Over the 1092 runs short_cost is fitted to, us summed:
+// this choice is 9 % below the fill's plan on average and 2 % above the best;
+// by the estimate alone 13 runs were over 6 % above the fill's plan, with the
+// margin 3.
+GemmPlan plan_gemm(const GemmTune& tune, int num_cu, int m, int n, int k, int x_dtype, const char* fname,
+                   size_t part_bytes) {
     const int cu = num_cu > 0 ? num_cu : 1;
+    const bool sk_ok = k % 128 == 0, few = m <= 32 && sk_ok;
     GemmPlan best{KB32, 1};
     double best_t = 1e30;
-    auto consider = [&](GemmKind kind) {
+    auto fits = [&](GemmKind kind, int s) {
         const bool sk = kind == KB16 || kind == KB16N;
         const int stages = sk ? k / 128 : k / 64;
+        return s == 1 || (kind < KB256 && stages % s == 0 && stages / s >= (sk ? 4 : 8) &&
+                          (size_t)s * m * n * 4 <= part_bytes);
+    };
+    const double* decode = few ? short_decode(fname) : nullptr;
+    auto cost = [&](GemmPlan p) {
+        return p.kind <= KB16N || (few && p.kind == KB32) ? short_cost(cu, p, m, n, k, x_dtype, decode)
+                                                          : plan_cost(cu, p, m, n, k, x_dtype, fname);
+    };
+    auto consider = [&](GemmKind kind) {
         for (int s : {1, 2, 4}) {
             if (tune.ksplit && s > 1) break;
-            if (tune.ksplit) s = tune.ksplit;
-            if (s > 1 &&
-                (kind >= KB256 || stages % s || stages / s < (sk ? 4 : 8) || (size_t)s * m * n * 4 > part_bytes)) {
-                if (!tune.ksplit) continue;
-                s = 1;
-            }
-            const double t = plan_cost(cu, GemmPlan{kind, s}, m, n, k, x_dtype, heavy);
+            if (tune.ksplit) s = fits(kind, tune.ksplit) ? tune.ksplit : 1;
+            if (!fits(kind, s)) continue;
+            const double t = cost(GemmPlan{kind, s});
             if (t < best_t) best_t = t, best = GemmPlan{kind, s};
         }
     };
-    const bool sk_ok = k % 128 == 0;
     if (tune.kind >= 0) {
         GemmKind kind = (GemmKind)tune.kind;
         if ((kind == KB16 || kind == KB16N) && !sk_ok) kind = KB32;
@@ -952,7 +1006,17 @@ GemmPlan plan_gemm(const GemmTune& tune, int num_cu, int m, int n, int k, int x_
         }
         return best;
     }
-    if (m <= 32 && sk_ok) {
+    if (few) {
+        const int wgs32 = (int)plan_wgs(GemmPlan{KB16, 1}, m, n, x_dtype);
+        GemmPlan fill{2LL * wgs32 <= cu ? KB16N : KB16, 1};
+        const int wgs = (int)plan_wgs(fill, m, n, x_dtype);
+        if (k <= 2048) fill.ksplit = 1;
+        else if (fill.kind == KB16) fill.ksplit = wgs <= cu ? 2 : 1;
+        else fill.ksplit = 4 * wgs <= cu ? 4 : (2 * wgs <= cu ? 2 : 1);
+        if (tune.ksplit) fill.ksplit = fits(fill.kind, tune.ksplit) ? tune.ksplit : 1;
+        while (!fits(fill.kind, fill.ksplit)) fill.ksplit /= 2;
+        best = fill, best_t = 0.88 * cost(fill);
+        if (!strcmp(fname, "f16w")) return best;
         consider(KB16);
         consider(KB16N);
     }
@@ -966,9 +1030,6 @@ GemmPlan plan_gemm(const GemmTune& tune, int num_cu, int m, int n, int k, int x_
     return best;
 }
 
-// formats whose decoding plan_cost charges for
-bool heavy_fmt(const char* name) { return !strcmp(name, "q5_k") || !strcmp(name, "q6_k"); }
-
 // Launches the planned tile kernel over Y[m, n] (row stride ldy).  plan_n:
 // the row count the plan is made for (a weight multiplied slice by slice
 // sums every slice in the same order).
@@ -976,7 +1037,7 @@ int gemm_launch(cima_hip_ctx* ctx, const char* fname, const void* x, const void*
                 int ldy, int x_dtype, int y_dtype, const GemmExt& gext, const char* api, float* part = nullptr,
                 size_t part_bytes = 0, int plan_n = 0) {
     const GemmPlan p = plan_gemm(GemmTune{ctx->tune_gemm_bn, ctx->tune_gemm_kind, ctx->tune_ksplit}, ctx->num_cu, m,
-                                 plan_n ? plan_n : n, k, x_dtype, heavy_fmt(fname), part ? part_bytes : 0);
+                                 plan_n ? plan_n : n, k, x_dtype, fname, part ? part_bytes : 0);
     const int bm = plan_bm(p.kind, x_dtype), bn = plan_bn(p.kind), ks = p.ksplit;
     const bool sk = p.kind == KB16 || p.kind == KB16N;
     static const char* const xn[] = {"f32", "f16", "bf16"};
@@ -1072,7 +1133,7 @@ int cima_hip_gemm_plan(int num_cu, int t, int m, int n, int k, int x_dtype, unsi
     if (num_cu <= 0 || m <= 0 || n <= 0 || k <= 0 || k % 64 || x_dtype < CIMA_DT_F32 || x_dtype > CIMA_DT_BF16)
         return fail(CIMA_E_INVALID, "%s: num_cu=%d m=%d n=%d k=%d x_dtype=%d", api, num_cu, m, n, k, x_dtype);
     if (!rows || !tokens || !ksplit) return fail(CIMA_E_INVALID, "%s: null pointer", api);
-    const GemmPlan p = plan_gemm(GemmTune{}, num_cu, m, n, k, x_dtype, F && heavy_fmt(F->name), (size_t)slab_bytes);
+    const GemmPlan p = plan_gemm(GemmTune{}, num_cu, m, n, k, x_dtype, F ? F->name : "nf4", (size_t)slab_bytes);
     *rows = plan_bm(p.kind, x_dtype), *tokens = plan_bn(p.kind), *ksplit = p.ksplit;
     return 0;
 }

@@ -30,6 +30,23 @@ def test_every_plan_can_run(t, xd):
                                        and 4 * ks * m * n <= slab)
 
 
+@pytest.mark.parametrize("t, m, n, k, xd, slab, plan", [
+    (12, 16, 1024, 4096, BF16, SLAB, (16, 16, 4)),   # 7.9 us; unsplit 9.1
+    (12, 16, 1024, 4096, F32, SLAB, (16, 16, 4)),    # 9.3; unsplit 12.9
+    (12, 16, 512, 2048, BF16, SLAB, (16, 16, 1)),    # 6.1; four ranges 6.6
+    (13, 16, 896, 4864, F16, SLAB, (16, 16, 2)),     # 9.4; 64 x 32 in four 12.4
+    (14, 24, 896, 4864, F16, SLAB, (16, 16, 2)),     # 64 x 32 in four 16.8 against 14.7
+    (3, 32, 4864, 896, F32, 0, (32, 16, 1)),         # 7.0; 16-row tiles 11.0
+    (0, 32, 4864, 896, F32, 0, (32, 16, 1)),         # 8.2; 16-row tiles 11.8
+    (12, 16, 14336, 4096, BF16, SLAB, (32, 16, 1)),  # 16.5
+    (12, 32, 14336, 4096, BF16, SLAB, (64, 32, 1)),  # 21.6; 16-token tiles 33.0
+    (12, 16, 4096, 14336, BF16, 0, (16, 16, 1))])    # 26.6; 32-row tiles 42.6
+def test_few_tokens_take_the_measured_plan(t, m, n, k, xd, slab, plan):
+    """Up to 32 tokens a plan by the CUs' fill stands unless another is clearly
+    cheaper (measured on MI355X, cold, us)."""
+    assert hip.gemm_plan(t, m, n, k, xd, slab) == plan
+
+
 def test_refusals():
     for bad in ((0, 16, 16, 256), (256, 0, 16, 256), (256, 16, 16, 100), (256, 16, 16, -256)):
         cu, m, n, k = bad
