@@ -941,6 +941,7 @@ struct GemmTune {
     int bn = 0;      // token tile, 0 = planned
     int kind = -1;   // GemmKind, before bn; -1 = none
     int ksplit = 0;  // 0 = planned, 1 = none, else this many where they divide and fit
+    unsigned kinds = ~0u;  // tiles the plan may take beyond 32 tokens, a bit for each kind
 };
 
 // The cheapest plan by its estimate: 16-token tiles up to 32 tokens, every
@@ -1020,24 +1021,45 @@ GemmPlan plan_gemm(const GemmTune& tune, int num_cu, int m, int n, int k, int x_
         consider(KB16);
         consider(KB16N);
     }
-    consider(KB32);
-    if (m > 32) consider(KB64);
-    if (m > 64) consider(KB128);
+    auto allowed = [&](GemmKind kind) {
+        if (few || (tune.kinds >> kind & 1)) consider(kind);
+    };
+    allowed(KB32);
+    if (m > 32) allowed(KB64);
+    if (m > 64) allowed(KB128);
     if (m > 128) {
-        consider(KB256);
-        if (x_dtype != CIMA_DT_F32) consider(KW256);
+        allowed(KB256);
+        if (x_dtype != CIMA_DT_F32) allowed(KW256);
     }
     return best;
 }
 
-// Launches the planned tile kernel over Y[m, n] (row stride ldy).  plan_n:
-// the row count the plan is made for (a weight multiplied slice by slice
-// sums every slice in the same order).
+// The plan of nr rows of an f16 weight of n rows that is multiplied slice by
+// slice.  The bits of Y must not depend on the slices, so only the slice's
+// rows choose among tiles that sum alike -- the 16-token ones; the group
+// tiles of four k groups; the one of two (f32 X at 128 tokens); the 256-token
+// ones -- and which of these it is follows from the rows that the
+// reference's 32 MiB slab holds.  Planned for all n rows, the tiles left most
+// CUs idle in each slice (measured on MI355X, NF4 of blocksize 48, 14336x4096
+// in slices of 4096 rows, us with the decoding, by n / by slices: 16 tokens,
+// f16 X, 257 / 231; 300, bf16 X, 473 / 326; 700 643 / 431).
+GemmPlan plan_slice(GemmTune tune, int num_cu, int m, int nr, int n, int k, int x_dtype) {
+    const int ref = (int)std::max(1LL, std::min((long long)n, (32LL << 20) / (2LL * k)));
+    const GemmKind kind = plan_gemm(tune, num_cu, m, ref, k, x_dtype, "f16w", 0).kind;
+    const bool two = x_dtype == CIMA_DT_F32;
+    tune.kinds = kind >= KB256 ? 1u << KB256 | 1u << KW256
+                 : kind == KB128 && two ? 1u << KB128 : 1u << KB32 | 1u << KB64 | (two ? 0u : 1u << KB128);
+    return plan_gemm(tune, num_cu, m, nr, k, x_dtype, "f16w", 0);
+}
+
+// Launches the planned tile kernel over Y[m, n] (row stride ldy); slice_of:
+// the rows of the f16 weight that these n rows are a slice of (0: none).
 int gemm_launch(cima_hip_ctx* ctx, const char* fname, const void* x, const void* w, void* y, int m, int n, int k,
                 int ldy, int x_dtype, int y_dtype, const GemmExt& gext, const char* api, float* part = nullptr,
-                size_t part_bytes = 0, int plan_n = 0) {
-    const GemmPlan p = plan_gemm(GemmTune{ctx->tune_gemm_bn, ctx->tune_gemm_kind, ctx->tune_ksplit}, ctx->num_cu, m,
-                                 plan_n ? plan_n : n, k, x_dtype, fname, part ? part_bytes : 0);
+                size_t part_bytes = 0, int slice_of = 0) {
+    const GemmTune tune{ctx->tune_gemm_bn, ctx->tune_gemm_kind, ctx->tune_ksplit};
+    const GemmPlan p = slice_of ? plan_slice(tune, ctx->num_cu, m, n, slice_of, k, x_dtype)
+                                : plan_gemm(tune, ctx->num_cu, m, n, k, x_dtype, fname, part ? part_bytes : 0);
     const int bm = plan_bm(p.kind, x_dtype), bn = plan_bn(p.kind), ks = p.ksplit;
     const bool sk = p.kind == KB16 || p.kind == KB16N;
     static const char* const xn[] = {"f32", "f16", "bf16"};
@@ -1128,12 +1150,15 @@ int cima_hip_set_gemm_plan(cima_hip_ctx* ctx, int rows, int tokens, int ksplit) 
 int cima_hip_gemm_plan(int num_cu, int t, int m, int n, int k, int x_dtype, unsigned long long slab_bytes, int* rows,
                        int* tokens, int* ksplit) {
     const char* api = "cima_hip_gemm_plan";
-    const Fmt* F = t ? fmt_of(t) : nullptr;
-    if (t && !F) return fail(CIMA_E_FORMAT, "%s: ggml type %d is not a supported GGUF block format", api, t);
+    const Fmt* F = t > 1 ? fmt_of(t) : nullptr;
+    if (t && t != 1 && !F) return fail(CIMA_E_FORMAT, "%s: ggml type %d is not a supported GGUF block format", api, t);
     if (num_cu <= 0 || m <= 0 || n <= 0 || k <= 0 || k % 64 || x_dtype < CIMA_DT_F32 || x_dtype > CIMA_DT_BF16)
         return fail(CIMA_E_INVALID, "%s: num_cu=%d m=%d n=%d k=%d x_dtype=%d", api, num_cu, m, n, k, x_dtype);
     if (!rows || !tokens || !ksplit) return fail(CIMA_E_INVALID, "%s: null pointer", api);
-    const GemmPlan p = plan_gemm(GemmTune{}, num_cu, m, n, k, x_dtype, F ? F->name : "nf4", (size_t)slab_bytes);
+    const int slice = (int)std::min((unsigned long long)n, slab_bytes / (2ULL * k));
+    if (t == 1 && slice < 1) return fail(CIMA_E_INVALID, "%s: a slab of %llu bytes holds no row", api, slab_bytes);
+    const GemmPlan p = t == 1 ? plan_slice(GemmTune{}, num_cu, m, slice, n, k, x_dtype)
+                              : plan_gemm(GemmTune{}, num_cu, m, n, k, x_dtype, F ? F->name : "nf4", (size_t)slab_bytes);
     *rows = plan_bm(p.kind, x_dtype), *tokens = plan_bn(p.kind), *ksplit = p.ksplit;
     return 0;
 }

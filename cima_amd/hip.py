@@ -193,7 +193,8 @@ def _act_of(t) -> int:
 
 def gemm_plan(fmt: int, m: int, n: int, k: int, x_dtype: int, slab_bytes: int = 0, num_cu: int = 256) -> tuple:
     """(tile rows, tile tokens, split along k) of a prefill product on a device of
-    ``num_cu`` compute units (cima_hip_gemm_plan; ``fmt`` 0: bitsandbytes)."""
+    ``num_cu`` compute units (cima_hip_gemm_plan; ``fmt`` 0: bitsandbytes, 1: f16
+    weights decoded into the slab)."""
     L = load_library()
     out = [ctypes.c_int() for _ in range(3)]
     rc = L.cima_hip_gemm_plan(num_cu, int(fmt), m, n, k, x_dtype, int(slab_bytes), *(ctypes.byref(v) for v in out))

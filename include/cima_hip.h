@@ -156,8 +156,9 @@ int cima_hip_set_gemm_plan(cima_hip_ctx* ctx, int rows, int tokens, int ksplit);
 /* The plan of a prefill product without overrides (no counterpart in the
  * reference): tile rows and tokens and the split along k that gguf_gemm
  * (slab_bytes 0) or gguf_gemm_slab takes on a device of num_cu compute
- * units.  ggml_type 0: bitsandbytes weights (nf4_gemm_slab, which never
- * splits).  Needs no device. */
+ * units.  ggml_type 0: bitsandbytes weights decoded in the tiles
+ * (nf4_gemm_slab, which never splits); 1: f16 weights decoded into the slab,
+ * the plan of a slice as large as the slab holds.  Needs no device. */
 int cima_hip_gemm_plan(int num_cu, int ggml_type, int m, int n, int k, int x_dtype, unsigned long long slab_bytes,
                        int* rows, int* tokens, int* ksplit);
 

@@ -47,6 +47,23 @@ def test_few_tokens_take_the_measured_plan(t, m, n, k, xd, slab, plan):
     assert hip.gemm_plan(t, m, n, k, xd, slab) == plan
 
 
+@pytest.mark.parametrize("xd", [F32, F16, BF16])
+def test_slices_are_planned_by_their_rows(xd):
+    """f16 weights of 14336 x 4096 in slices of 4096 rows: at least a quarter of
+    the 256 compute units at work up to 64 tokens, over half beyond 200 (planned
+    for the whole weight, the 256-token tiles left 32 workgroups at 300
+    tokens); every slab size sums alike."""
+    for m in (16, 64, 200, 300, 700):
+        rows, tokens, ks = hip.gemm_plan(1, m, 14336, 4096, xd, SLAB)
+        assert ks == 1 and -(-4096 // rows) * -(-m // tokens) >= (64 if m <= 64 else 128 if m != 700 else 96)
+        alike = {t for t in TILES if [t[1] == 16, t[1] == 256, t == (128, 128)] ==
+                 [tokens == 16, tokens == 256, (rows, tokens) == (128, 128)]}
+        assert all(hip.gemm_plan(1, m, 14336, 4096, xd, s)[:2] in alike
+                   for s in (8192, 100 << 10, 1 << 20, SLAB, 1 << 30))
+    with pytest.raises(hip.EngineError):
+        hip.gemm_plan(1, 16, 14336, 4096, xd, 8191)
+
+
 def test_refusals():
     for bad in ((0, 16, 16, 256), (256, 0, 16, 256), (256, 16, 16, 100), (256, 16, 16, -256)):
         cu, m, n, k = bad

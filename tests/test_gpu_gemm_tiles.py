@@ -128,6 +128,28 @@ def test_bitsandbytes_on_every_tile(hip, rows, tokens, bs):
         assert rel(y.float().cpu().numpy(), want) <= (1e-5 if yd == F32 else 2.0 ** -11), (xd, yd)
 
 
+@pytest.mark.parametrize("m", [13, 32, 40, 100, 140, 600, 2100])
+@pytest.mark.parametrize("k", [768, 320])
+def test_f16_slices_sum_alike(hip, m, k):
+    """Weights decoded into the slab a slice at a time: slices of whatever size
+    the slab holds, the last one short, take tiles by their own rows, and Y has
+    the bits of one slice of all rows."""
+    n, bs = 1030, 48 if k % 48 == 0 else 80
+    rng = np.random.default_rng(m + k)
+    p, a, q = (torch.from_numpy(v).cuda() for v in (rng.integers(0, 256, n * k // 2, dtype=np.uint8),
+                                                    (rng.random(-(-n * k // bs)) + 0.01).astype(np.float32),
+                                                    nf4.NF4_CODE.copy()))
+    for xd, yd in ((BF16, F32), (F16, F16), (F32, F32)):
+        x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(TDT[xd]).cuda()
+        ys = []
+        for rows in (n, 512, 130, 24):
+            slab = torch.empty(2 * rows * k, dtype=torch.uint8, device="cuda")
+            ys.append(torch.full((m, n), float("nan"), dtype=TDT[yd], device="cuda"))
+            hip.nf4_gemm_slab(x, p, a, q, ys[-1], m, n, k, bs, slab)
+        torch.cuda.synchronize()
+        assert bool(torch.isfinite(ys[0]).all()) and all(torch.equal(y, ys[0]) for y in ys[1:]), (xd, yd)
+
+
 @pytest.mark.parametrize("t", [Q8_0, Q4_0, Q5_0, Q6_K])
 @pytest.mark.parametrize("tile", [16, 32, 64, 128, 256])
 def test_weights_two_bytes_off_a_word(hip, t, tile):
