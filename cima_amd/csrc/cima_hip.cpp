@@ -172,7 +172,9 @@ bool gemm_b16l(const char* weights, const char* xt) {
 
 // decode-step kernels (cima_decode.hsaco)
 const char* const kDecodeKernels[] = {
-    "cima_rmsnorm_f16",     "cima_rope_f16",        "cima_kv_append_f16",    "cima_attn_split_d64",
+    "cima_rmsnorm_f16",     "cima_rmsnorm_f16_w1",  "cima_rmsnorm_f16_w4",   "cima_rope_f16",
+    "cima_kv_append_f16",
+    "cima_attn_split_d64",
     "cima_attn_reduce_d64", "cima_attn_split_d128", "cima_attn_reduce_d128", "cima_attn_decode_d64_c64",
     "cima_attn_decode_d64_c128", "cima_attn_decode_d64_c256", "cima_attn_decode_d128_c64",
     "cima_attn_decode_d128_c128", "cima_attn_decode_d128_c256", "cima_argmax_f16", "cima_argmax_to_ids",
@@ -1233,6 +1235,11 @@ int attn_dim_ok(int dim) { return dim == 64 || dim == 128; }
 // positions per attention chunk the kernels stage at most (ATT_MAX_CSZ)
 const int kAttMaxChunk = 256;
 
+// longest rows of cima_rmsnorm_f16_w1 and _w4 (256 threads of one or four
+// 8-element words), and the shortest: below it the pass of single elements is
+// no slower (decode_ops.hip)
+const int kRmsWordsFrom = 256, kRmsOneWord = 2048, kRmsFourWords = 8192;
+
 // heads per workgroup of cima_rope_f16 (ROPE_HEADS in decode_ops.hip)
 const int kRopeHeads = 16;
 
@@ -1281,7 +1288,10 @@ int cima_hip_rmsnorm(cima_hip_ctx* ctx, const void* x, const void* w, void* y, i
     if (rows == 0) return 0;
     if (!x || !y) return fail(CIMA_E_INVALID, "%s: null x or y", kApiRms);
     void* args[] = {&x, &w, &y, &n, &eps};
-    return launch_named(ctx, "cima_rmsnorm_f16", (unsigned)rows, 256, args, kApiRms);
+    const bool words = n >= kRmsWordsFrom && n <= kRmsFourWords && n % 8 == 0 && aligned(x, 16) && aligned(w, 16) &&
+                       aligned(y, 16);
+    return launch_named(ctx, !words ? "cima_rmsnorm_f16" : n <= kRmsOneWord ? "cima_rmsnorm_f16_w1" : "cima_rmsnorm_f16_w4",
+                        (unsigned)rows, 256, args, kApiRms);
 }
 
 int cima_hip_rope(cima_hip_ctx* ctx, void* x, int rows, int heads, int dim, int pos0, float theta, int nfreqs,

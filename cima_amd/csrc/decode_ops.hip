@@ -22,77 +22,91 @@ DEV float wave_max(float v) { return wave_max_u(v); }
 
 // y[row] = f16(sat(x) * rsqrt(mean(sat(x)^2) + eps) * w); w may be null
 // (unit weight).  One 256-thread workgroup per row (k_rmsnorm,
-// src/kernels.cu:37-50).  Rows of up to 8192 elements, a multiple of 8 and
-// 16-byte aligned, stay in registers between the sum and the scaling, in
-// 16-byte words all loaded at once; any other row takes the two scalar
-// passes.  Bound by one memory round trip and the launch (measured on
-// MI355X, 585 rows of 4096 already in the caches: 11.9 -> 4.6 us).
-constexpr int RMS_WORDS = 4;  // 16-byte words per thread held in registers
+// src/kernels.cu:37-50).  _w1, _w4: rows that are a multiple of 8 elements
+// and 16-byte aligned, at most 2048 and 8192, stay in registers between the
+// sum and the scaling, in one or four 16-byte words a thread, all loaded at
+// once.  Without suffix: two passes of single elements, for any row, and the
+// faster one below 256 elements.  Bound by one memory round trip and the
+// launch.  Measured on MI355X in the caches, single elements / words, us: 585
+// rows of 4096 8.16 / 3.79, of 896 3.43 / 2.31, of 256 2.26 / 2.14, of 64 2.14
+// / 2.25; 4096 rows of 4096 26.5 / 11.5, of 896 7.17 / 4.76, of 256 4.21 /
+// 3.76, of 128 3.45 / 3.74, of 64 2.96 / 3.67.  (Four words at every length
+// cost as much for 64 elements as for 896: 4096 rows 7.6 and 8.3.)
+DEV float rms_inv(float ss, int n, float eps) {
+    __shared__ float red[4];
+    ss = wave_sum(ss);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    return 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)n + eps);
+}
 extern "C" __global__ __launch_bounds__(256) void cima_rmsnorm_f16(const uint16_t* __restrict__ x,
                                                                    const uint16_t* __restrict__ w,
                                                                    uint16_t* __restrict__ y, int n, float eps) {
-    __shared__ float red[4];
     const uint16_t* xr = x + (size_t)blockIdx.x * n;
     uint16_t* yr = y + (size_t)blockIdx.x * n;
-    const bool vec = (n & 7) == 0 && n <= 256 * 8 * RMS_WORDS &&
-                     ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
-                       reinterpret_cast<uintptr_t>(y)) & 15) == 0;
-    auto total = [&](float ss) {
-        ss = wave_sum(ss);
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-        __syncthreads();
-        return 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)n + eps);
-    };
-    if (vec) {
-        const int nv = n >> 3;
-        uint4 xv[RMS_WORDS], wv[RMS_WORDS];
-        float ss = 0.f;
-#pragma unroll
-        for (int j = 0; j < RMS_WORDS; j++) {
-            const int i = threadIdx.x + 256 * j;
-            xv[j] = make_uint4(0, 0, 0, 0);
-            wv[j] = make_uint4(0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u);
-            if (i < nv) {
-                xv[j] = reinterpret_cast<const uint4*>(xr)[i];
-                if (w) wv[j] = reinterpret_cast<const uint4*>(w)[i];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < RMS_WORDS; j++) {
-            const uint32_t u[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float a = sat16(h2f(u[e] & 0xffffu)), b = sat16(h2f(u[e] >> 16));
-                ss += a * a;
-                ss += b * b;
-            }
-        }
-        const float inv = total(ss);
-#pragma unroll
-        for (int j = 0; j < RMS_WORDS; j++) {
-            const int i = threadIdx.x + 256 * j;
-            if (i >= nv) continue;
-            const uint32_t u[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
-            const uint32_t g[4] = {wv[j].x, wv[j].y, wv[j].z, wv[j].w};
-            uint32_t o[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                o[e] = f2h2(sat16(h2f(u[e] & 0xffffu)) * inv * h2f(g[e] & 0xffffu),
-                            sat16(h2f(u[e] >> 16)) * inv * h2f(g[e] >> 16));
-            reinterpret_cast<uint4*>(yr)[i] = make_uint4(o[0], o[1], o[2], o[3]);
-        }
-        return;
-    }
     float ss = 0.f;
     for (int i = threadIdx.x; i < n; i += 256) {
         const float v = sat16(h2f(xr[i]));
         ss += v * v;
     }
-    const float inv = total(ss);
+    const float inv = rms_inv(ss, n, eps);
     for (int i = threadIdx.x; i < n; i += 256) {
         const float g = w ? h2f(w[i]) : 1.0f;
         yr[i] = (uint16_t)f2h(sat16(h2f(xr[i])) * inv * g);
     }
+}
+template <int W>
+DEV void rms_words(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, uint16_t* __restrict__ y, int n,
+                   float eps) {
+    const uint16_t* xr = x + (size_t)blockIdx.x * n;
+    uint16_t* yr = y + (size_t)blockIdx.x * n;
+    const int nv = n >> 3;
+    uint4 xv[W], wv[W];
+#pragma unroll
+    for (int j = 0; j < W; j++) {
+        const int i = threadIdx.x + 256 * j;
+        xv[j] = make_uint4(0, 0, 0, 0);
+        wv[j] = make_uint4(0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u);
+        if (i < nv) {
+            xv[j] = reinterpret_cast<const uint4*>(xr)[i];
+            if (w) wv[j] = reinterpret_cast<const uint4*>(w)[i];
+        }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < W; j++) {
+        const uint32_t u[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float a = sat16(h2f(u[e] & 0xffffu)), b = sat16(h2f(u[e] >> 16));
+            ss += a * a;
+            ss += b * b;
+        }
+    }
+    const float inv = rms_inv(ss, n, eps);
+#pragma unroll
+    for (int j = 0; j < W; j++) {
+        const int i = threadIdx.x + 256 * j;
+        if (i >= nv) continue;
+        const uint32_t u[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
+        const uint32_t g[4] = {wv[j].x, wv[j].y, wv[j].z, wv[j].w};
+        uint32_t o[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            o[e] = f2h2(sat16(h2f(u[e] & 0xffffu)) * inv * h2f(g[e] & 0xffffu),
+                        sat16(h2f(u[e] >> 16)) * inv * h2f(g[e] >> 16));
+        reinterpret_cast<uint4*>(yr)[i] = make_uint4(o[0], o[1], o[2], o[3]);
+    }
+}
+extern "C" __global__ __launch_bounds__(256) void cima_rmsnorm_f16_w1(const uint16_t* __restrict__ x,
+                                                                      const uint16_t* __restrict__ w,
+                                                                      uint16_t* __restrict__ y, int n, float eps) {
+    rms_words<1>(x, w, y, n, eps);
+}
+extern "C" __global__ __launch_bounds__(256) void cima_rmsnorm_f16_w4(const uint16_t* __restrict__ x,
+                                                                      const uint16_t* __restrict__ w,
+                                                                      uint16_t* __restrict__ y, int n, float eps) {
+    rms_words<4>(x, w, y, n, eps);
 }
 
 // --------------------------------------------------------------------- RoPE

@@ -17,7 +17,8 @@ def dev(a, offset=0):
     return t[offset:]
 
 
-@pytest.mark.parametrize("n, offset", [(8, 0), (2048, 0), (2056, 0), (8192, 0), (8200, 0), (100, 0), (4096, 1)])
+@pytest.mark.parametrize("n, offset", [(8, 0), (248, 0), (256, 0), (1000, 0), (2048, 0), (2056, 0), (8192, 0),
+                                       (8200, 0), (100, 0), (4096, 1)])
 @pytest.mark.parametrize("unit", [False, True])
 def test_rmsnorm_rows(hip, n, offset, unit):
     """Within two f16 steps of float64 (one rounding, and the inverse root
