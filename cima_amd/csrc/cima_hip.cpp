@@ -173,7 +173,7 @@ bool gemm_b16l(const char* weights, const char* xt) {
 // decode-step kernels (cima_decode.hsaco)
 const char* const kDecodeKernels[] = {
     "cima_rmsnorm_f16",     "cima_rmsnorm_f16_w1",  "cima_rmsnorm_f16_w4",   "cima_rope_f16",
-    "cima_kv_append_f16",
+    "cima_rope_f16_g",      "cima_kv_append_f16",
     "cima_attn_split_d64",
     "cima_attn_reduce_d64", "cima_attn_split_d128", "cima_attn_reduce_d128", "cima_attn_decode_d64_c64",
     "cima_attn_decode_d64_c128", "cima_attn_decode_d64_c256", "cima_attn_decode_d128_c64",
@@ -1240,8 +1240,10 @@ const int kAttMaxChunk = 256;
 // no slower (decode_ops.hip)
 const int kRmsWordsFrom = 256, kRmsOneWord = 2048, kRmsFourWords = 8192;
 
-// heads per workgroup of cima_rope_f16 (ROPE_HEADS in decode_ops.hip)
-const int kRopeHeads = 16;
+// heads per workgroup of cima_rope_f16_g (ROPE_HEADS in decode_ops.hip), and
+// where it is taken: from kRopeRowHeads heads of all rows on, with more heads
+// in a row than a workgroup takes at a time
+const int kRopeHeads = 16, kRopeRowHeads = 3072, kRopeAtATime = 4;
 
 // threads of cima_attn_reduce_d<dim> (ATT_MERGE_T in decode_ops.hip)
 const int kAttMergeThreads = 1024;
@@ -1303,8 +1305,10 @@ int cima_hip_rope(cima_hip_ctx* ctx, void* x, int rows, int heads, int dim, int 
     if (rows == 0) return 0;
     if (!x) return fail(CIMA_E_INVALID, "%s: null x", api);
     void* args[] = {&x, &heads, &dim, &pos0, &theta, &nfreqs, &pos_dev};
+    if ((long long)rows * heads < kRopeRowHeads || heads <= kRopeAtATime)
+        return launch_named(ctx, "cima_rope_f16", (unsigned)(rows * heads), 64, args, api);
     const long long hgs = (heads + kRopeHeads - 1) / kRopeHeads;
-    return launch_named(ctx, "cima_rope_f16", (unsigned)(rows * hgs), 256, args, api);
+    return launch_named(ctx, "cima_rope_f16_g", (unsigned)(rows * hgs), 256, args, api);
 }
 
 int cima_hip_kv_append(cima_hip_ctx* ctx, const void* k, const void* v, void* kc, void* vc, int rows, int kv_heads,

@@ -123,15 +123,36 @@ DEV void rope_rot_f(float a, float b, float p, float freq, float& oa, float& ob)
 
 // In place over x [rows, heads, dim]: row r sits at position pos0 + r, or
 // *pos_dev + r when pos_dev is set (graph replay).  Pairs i >= nfreqs pass
-// through.  Grid rows * ceil(heads / ROPE_HEADS): a 256-thread workgroup
-// takes up to ROPE_HEADS heads of a row, four at a time, so that a pair's
-// power, sine and cosine -- what the kernel spends its time on -- are
-// computed once per thread for up to four heads (measured on MI355X, 585
-// rows of 32 heads of 128: 9.9 -> 6.3 us).
+// through.  A head of a row per 64-thread workgroup.
+extern "C" __global__ __launch_bounds__(64) void cima_rope_f16(uint16_t* __restrict__ x, int heads, int dim,
+                                                               int pos0, float theta, int nfreqs,
+                                                               const int* __restrict__ pos_dev) {
+    const int row = blockIdx.x / heads, h = blockIdx.x % heads;
+    if (pos_dev) pos0 = *pos_dev;
+    uint16_t* v = x + ((size_t)row * heads + h) * dim;
+    const float p = (float)(pos0 + row);
+    const int half = dim >> 1;
+    for (int i = threadIdx.x; i < half && i < nfreqs; i += 64) {
+        float oa, ob;
+        rope_rot_f(h2f(v[i]), h2f(v[i + half]), p, rope_freq(i, dim, theta), oa, ob);
+        v[i] = (uint16_t)f2h(oa);
+        v[i + half] = (uint16_t)f2h(ob);
+    }
+}
+
+// The same with up to ROPE_HEADS heads of a row per 256-thread workgroup,
+// four at a time (grid rows * ceil(heads / ROPE_HEADS)), so that a pair's
+// power, sine and cosine -- what the kernels spend their time on -- are
+// computed once per thread for up to four heads.  It pays where the other's
+// workgroups fill the CUs several times over and a thread has more than one
+// head.  Measured on MI355X in the caches, a head / up to 16 per workgroup,
+// us: 585 rows of 32 heads of 128 8.3 / 4.8, of 8 3.65 / 3.24, of 5 3.06 /
+// 3.05, of 2 2.43 / 2.81; 64 rows of 64 3.38 / 2.98, of 32 2.67 / 2.89; 4096 of
+// 1 3.35 / 6.74; one row of 32 2.13 / 2.65.
 constexpr int ROPE_HEADS = 16;
-extern "C" __global__ __launch_bounds__(256) void cima_rope_f16(uint16_t* __restrict__ x, int heads, int dim,
-                                                                int pos0, float theta, int nfreqs,
-                                                                const int* __restrict__ pos_dev) {
+extern "C" __global__ __launch_bounds__(256) void cima_rope_f16_g(uint16_t* __restrict__ x, int heads, int dim,
+                                                                  int pos0, float theta, int nfreqs,
+                                                                  const int* __restrict__ pos_dev) {
     const int hgs = (heads + ROPE_HEADS - 1) / ROPE_HEADS;
     const int row = blockIdx.x / hgs, h0 = (blockIdx.x % hgs) * ROPE_HEADS, h1 = min(h0 + ROPE_HEADS, heads);
     if (pos_dev) pos0 = *pos_dev;

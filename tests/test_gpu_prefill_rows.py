@@ -38,10 +38,12 @@ def test_rmsnorm_rows(hip, n, offset, unit):
 
 @pytest.mark.parametrize("heads, dim, nfreqs", [(1, 64, 32), (15, 64, 32), (16, 128, 64), (17, 128, 64), (33, 32, 10),
                                                 (2, 256, 128)])
-def test_rope_head_counts(hip, heads, dim, nfreqs):
-    """Every head of every row rotates once: against the oracle row by row
-    (fp32 sine and cosine of fp32 angles below 2000 rad: absolute 2e-3)."""
-    rows, pos = 5, 1000
+@pytest.mark.parametrize("rows", [5, 205])
+def test_rope_head_counts(hip, heads, dim, nfreqs, rows):
+    """Every head of every row rotates once, by a head or by up to 16 heads a
+    workgroup (from 3072 heads on): against the oracle row by row (fp32 sine
+    and cosine of fp32 angles below 2000 rad: absolute 2e-3)."""
+    pos = 1000
     x = np.random.default_rng(heads).normal(size=(rows, heads, dim)).astype(np.float16)
     t = dev(x)
     hip.rope(t, rows, heads, dim, pos, 1e4, nfreqs)
