@@ -178,7 +178,7 @@ const char* const kDecodeKernels[] = {
     "cima_attn_reduce_d64", "cima_attn_split_d128", "cima_attn_reduce_d128", "cima_attn_decode_d64_c64",
     "cima_attn_decode_d64_c128", "cima_attn_decode_d64_c256", "cima_attn_decode_d128_c64",
     "cima_attn_decode_d128_c128", "cima_attn_decode_d128_c256", "cima_argmax_f16", "cima_argmax_to_ids",
-    "cima_pos_bump"};
+    "cima_pos_bump", "cima_attn_reduce_wide_d64", "cima_attn_reduce_wide_d128"};
 
 std::string default_code_dir() {
     Dl_info info;
@@ -1245,8 +1245,10 @@ const int kRmsWordsFrom = 256, kRmsOneWord = 2048, kRmsFourWords = 8192;
 // in a row than a workgroup takes at a time
 const int kRopeHeads = 16, kRopeRowHeads = 3072, kRopeAtATime = 4;
 
-// threads of cima_attn_reduce_d<dim> (ATT_MERGE_T in decode_ops.hip)
-const int kAttMergeThreads = 1024;
+// threads of cima_attn_reduce_wide_d<dim> (ATT_MERGE_T in decode_ops.hip), and
+// the most live chunks that are merged by a thread per element instead (the
+// two are even at about 25, decode_ops.hip)
+const int kAttMergeThreads = 1024, kAttMergeFew = 24;
 
 // query heads per workgroup of cima_attn_decode_d<dim>_c<cp> (AT_GMAX in
 // decode_ops.hip; 4 cp threads, chunks of up to cp positions) and its LDS
@@ -1348,10 +1350,15 @@ int cima_hip_attn_reduce(cima_hip_ctx* ctx, const float* part, void* out, int q_
         return fail(CIMA_E_INVALID, "%s: q_heads=%d dim=%d csz=%d n_chunks=%d seq=%d", api, q_heads, dim, csz,
                     n_chunks, seq);
     if (!part || !out) return fail(CIMA_E_INVALID, "%s: null pointer", api);
+    // the most chunks that can be live: a position on the device is not known
+    const int len = pos_dev ? max_seq : std::min(seq, max_seq);
+    long long live = std::min((long long)n_chunks, ((long long)len + csz - 1) / csz);
+    if (window > 0) live = std::min(live, ((long long)window + csz - 1) / csz + 1);
+    const bool few = live <= kAttMergeFew;
     char name[48];
-    snprintf(name, sizeof name, "cima_attn_reduce_d%d", dim);
+    snprintf(name, sizeof name, "cima_attn_reduce_%sd%d", few ? "" : "wide_", dim);
     void* args[] = {&part, &out, &csz, &n_chunks, &seq, &max_seq, &window, &pos_dev};
-    return launch_named(ctx, name, (unsigned)q_heads, kAttMergeThreads, args, api);
+    return launch_named(ctx, name, (unsigned)q_heads, few ? dim : kAttMergeThreads, args, api);
 }
 
 int cima_hip_attn_decode_noalloc(cima_hip_ctx* ctx, const void* q, const void* kc, const void* vc, void* out,
@@ -1468,7 +1475,9 @@ int cima_hip_decode_step(cima_hip_ctx* ctx, const cima_decoder* d) {
     // layers (4 of them, Q4_K) at position 10 of 1024 (133 KB) 217 / 194, 1000
     // of 2048 226 / 198, 10 of 8192 245 / 211, 8000 of 8192 373 / 220;
     // Qwen2.5-0.5B (24 layers, Q8_0) at 10 of 4096 (118 KB) 617 / 623, 2047
-    // of 4096 631 / 652, 10 of 8192 620 / 628, 8000 of 8192 798 / 666.
+    // of 4096 631 / 652, 10 of 8192 620 / 628, 2000 of 8192 608 / 628, 8000 of
+    // 8192 798 / 666: a small model with a long cache pays 1-3 % up to about
+    // position 3000 for 17 % at 8000.
     // Rows of q past 16384 elements keep the fused launch and its LDS limit.
     const bool merge_apart = (size_t)d->q_heads * nch * (hd + 2) * 4 > (128u << 10) && qd <= 16384;
     if (!aligned(d->part, 8)) return fail(CIMA_E_INVALID, "%s: partials must be 8-byte aligned", api);

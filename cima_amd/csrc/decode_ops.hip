@@ -330,22 +330,42 @@ DEV void attn_chunk(AttnLds<D>& L, const AttnRegs<D>& R, int s0, int s1, int sne
 }
 
 // Merge chunks [c0, active) of one head: out = sum_c e^(m_c - M) acc_c /
-// sum_c e^(m_c - M) l_c (k_attn_reduce, src/kernels.cu:614-639).  1024
-// threads: group t / D takes chunks c0 + t / D + j 1024 / D, thread t %
-// D of it one output element, eight chunks' loads in flight at a time under
-// a running maximum, and the groups' sums are rescaled to the common
-// maximum and added in group order.  Bound by the latency of one or two
-// memory round trips: one 256-thread workgroup walking every chunk in turn
-// had a serial exponential chain per chunk (measured on MI355X, 63 chunks
-// of 32 heads of 128: 6.5 -> 3.7 us).
-constexpr int ATT_MERGE_T = 1024;
+// sum_c e^(m_c - M) l_c (k_attn_reduce, src/kernels.cu:614-639), with a
+// running maximum so every chunk is read once.  D threads, an output element
+// each.  The maximum starts at the lowest finite value: a chunk
+// whose own is -inf (nothing unmasked in it) then takes the weight e^-inf =
+// 0 wherever it stands.
 template <int D>
 DEV void attn_merge(const float* __restrict__ ph, int c0, int active, uint16_t* __restrict__ oh) {
+    const int t = threadIdx.x;
+    float M = -3.402823466e38f, Ls = 0.f, a = 0.f;
+#pragma unroll 4
+    for (int c = c0; c < active; c++) {
+        const float* pc = ph + (size_t)c * (D + 2);
+        const float m = pc[0], l = pc[1], v = pc[2 + t];
+        const float Mn = fmaxf(M, m);
+        const float so = __expf(M - Mn), sn = __expf(m - Mn);
+        Ls = Ls * so + l * sn;
+        a = a * so + v * sn;
+        M = Mn;
+    }
+    oh[t] = (uint16_t)f2h(a / Ls);
+}
+
+// The same by 1024 threads, for many chunks: group t / D takes chunks c0 + t /
+// D + j 1024 / D, thread t % D of it one output element, eight chunks' loads
+// in flight at a time under a running maximum, and the groups' sums are
+// rescaled to the common maximum and added in group order.  Bound by the
+// latency of one or two memory round trips, where the other has a serial
+// exponential chain per chunk.  Measured on MI355X in the caches, 32 heads of
+// 128, us, D / 1024 threads per head: 4 chunks 2.0 / 2.7, 16 2.7 /
+// 3.3, 33 3.8 / 3.3, 64 5.9 / 3.3, 128 10.2 / 4.6.
+constexpr int ATT_MERGE_T = 1024;
+template <int D>
+DEV void attn_merge_wide(const float* __restrict__ ph, int c0, int active, uint16_t* __restrict__ oh) {
     constexpr int G = ATT_MERGE_T / D, B = 8;
     __shared__ float sm[G], sl[G], sa[G][D];
     const int g = threadIdx.x / D, t = threadIdx.x % D;
-    // the lowest finite start: a chunk whose maximum is -inf (nothing unmasked
-    // in it) then takes the weight e^-inf = 0 wherever it stands
     float M = -3.402823466e38f, Ls = 0.f, a = 0.f;
     for (int c = c0 + g; c < active; c += G * B) {
         float m[B], l[B], v[B];
@@ -422,14 +442,16 @@ DEV void attn_split_body(const uint16_t* __restrict__ q, const uint16_t* __restr
     attn_chunk<D>(L, R, s0, s1, -1, scale, part + ((size_t)h * n_chunks + ci) * (D + 2));
 }
 
-template <int D>
+template <int D, bool WIDE>
 DEV void attn_reduce_body(const float* __restrict__ part, uint16_t* __restrict__ out, int csz, int n_chunks,
                           int seq, int max_seq, int window, const int* __restrict__ pos_dev) {
     int wlo;
     attn_range(seq, max_seq, window, pos_dev, wlo);
     const int h = blockIdx.x;
     const int active = min((seq + csz - 1) / csz, n_chunks);
-    attn_merge<D>(part + (size_t)h * n_chunks * (D + 2), wlo / csz, active, out + (size_t)h * D);
+    const float* ph = part + (size_t)h * n_chunks * (D + 2);
+    if constexpr (WIDE) attn_merge_wide<D>(ph, wlo / csz, active, out + (size_t)h * D);
+    else attn_merge<D>(ph, wlo / csz, active, out + (size_t)h * D);
 }
 
 // Decode attention partials of one layer at position pos = *pos_dev, with
@@ -729,10 +751,15 @@ DEV void attn_fused_body(const uint16_t* __restrict__ qkv, uint16_t* __restrict_
         attn_split_body<D>(q, kc, vc, part, q_heads, kv_heads, seq, max_seq, csz, n_chunks, scale, window,       \
                            pos_dev);                                                                             \
     }                                                                                                            \
-    extern "C" __global__ __launch_bounds__(ATT_MERGE_T) void cima_attn_reduce_d##D(                              \
+    extern "C" __global__ __launch_bounds__(D) void cima_attn_reduce_d##D(                                       \
         const float* part, uint16_t* out, int csz, int n_chunks, int seq, int max_seq, int window,               \
         const int* pos_dev) {                                                                                    \
-        attn_reduce_body<D>(part, out, csz, n_chunks, seq, max_seq, window, pos_dev);                            \
+        attn_reduce_body<D, false>(part, out, csz, n_chunks, seq, max_seq, window, pos_dev);                     \
+    }                                                                                                            \
+    extern "C" __global__ __launch_bounds__(ATT_MERGE_T) void cima_attn_reduce_wide_d##D(                         \
+        const float* part, uint16_t* out, int csz, int n_chunks, int seq, int max_seq, int window,               \
+        const int* pos_dev) {                                                                                    \
+        attn_reduce_body<D, true>(part, out, csz, n_chunks, seq, max_seq, window, pos_dev);                      \
     }                                                                                                            \
     ATTN_FUSED(D, 64) ATTN_FUSED(D, 128) ATTN_FUSED(D, 256)
 

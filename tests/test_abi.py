@@ -76,7 +76,7 @@ def test_decode_object_holds_every_kernel():
     blob = open(cbuild.HSACOS["decode"], "rb").read()
     names = ["cima_rmsnorm_f16", "cima_rmsnorm_f16_w1", "cima_rmsnorm_f16_w4", "cima_rope_f16", "cima_rope_f16_g",
              "cima_kv_append_f16", "cima_argmax_f16", "cima_argmax_to_ids", "cima_pos_bump"]
-    names += [f"cima_attn_{k}_d{d}" for k in ("split", "reduce", "decode") for d in (64, 128)]
+    names += [f"cima_attn_{k}_d{d}" for k in ("split", "reduce", "reduce_wide", "decode") for d in (64, 128)]
     for n in names:
         assert n.encode() in blob, n
 

@@ -12,8 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dim", [64, 128])
-@pytest.mark.parametrize("seq, window", [(1, 0), (16, 0), (17, 0), (127, 0), (128, 0), (129, 0), (1024, 0), (1025, 0),
-                                         (2100, 0), (2100, 33), (2100, 700)])
+@pytest.mark.parametrize("seq, window", [(1, 0), (16, 0), (17, 0), (127, 0), (128, 0), (129, 0), (384, 0), (385, 0),
+                                         (1024, 0), (1025, 0), (2100, 0), (2100, 33), (2100, 700)])
 def test_attn_reduce_chunk_counts(hip, dim, seq, window):
     """1 to 132 chunks of 16 positions against the merge in float64; chunks
     outside the live range hold NaN and must not be read into the result.
