@@ -307,8 +307,8 @@ struct GemmExt {
 // nonzero ones may lose bits (f16 subnormals step by 2^-24).  f32 X is
 // rounded anyway (the 1e-3 bar), but |x| >= 65520 becomes inf too.  Every
 // workgroup checks its own 1/(grid size) share of X once (XScan: a few
-// 16-byte words per thread) and ORs
-// flags into a word of this code object, which the host reads back on
+// 16-byte words per thread) and ORs flags into a word of device memory
+// (cima_gemm_status in gguf_gemm.hip), which the host reads back on
 // request (cima_hip_gemm_status): bit 0 = values beyond f16's range, or not
 // finite; bit 1 = nonzero bf16 values below 2^-17.  The loads go out after
 // the main loop, beside the output stores, and are checked last.  Measured
@@ -317,7 +317,6 @@ struct GemmExt {
 // checked before the main loop instead it cost 1.3-2.6 us at 16-32
 // tokens, and inside the tiles' own conversions every stage (+1170 VALU
 // instructions in the 256-token tile, 102 -> 150 us at 512 tokens).
-__device__ unsigned cima_gemm_status;
 struct XRange {
     // one word of flags, two bf16 halves at a time (magnitudes h <= 0x7fff,
     // so the additions below never carry out of a half): bit 15 of a half

@@ -41,6 +41,25 @@ DEV void store4(void* y, float4_t o, int tok, int row, int m, int n, int ldy, bo
     }
 }
 
+// 16 bytes of X to LDS as f16: eight elements, four of f32
+template <int XT>
+DEV void store_x(uint16_t* dst, uint4 x) {
+    const uint32_t v[4] = {x.x, x.y, x.z, x.w};
+    if constexpr (XT == XT_F16) {
+        *reinterpret_cast<uint4*>(dst) = x;
+    } else if constexpr (XT == XT_BF16) {
+        uint32_t o[4];
+        static_for<4>([&](auto E) INL {
+            o[E] = pack_f16(__builtin_bit_cast(float, v[E] << 16), __builtin_bit_cast(float, v[E] & 0xffff0000u));
+        });
+        *reinterpret_cast<uint4*>(dst) = make_uint4(o[0], o[1], o[2], o[3]);
+    } else {
+        *reinterpret_cast<uint2*>(dst) =
+            make_uint2(pack_f16(__builtin_bit_cast(float, v[0]), __builtin_bit_cast(float, v[1])),
+                       pack_f16(__builtin_bit_cast(float, v[2]), __builtin_bit_cast(float, v[3])));
+    }
+}
+
 // Group tiles (17 to about 256 tokens): 64 weight rows x T = 32, 64 or 128
 // tokens in 8 waves.  Four k groups of two waves take every fourth 64-k
 // stage each; a wave owns 32 rows and all T tokens of its group's stages,
@@ -53,7 +72,8 @@ DEV void store4(void* y, float4_t o, int tok, int row, int m, int n, int ldy, bo
 // so its B fragment is x[32h + 8q, +8) of token l % 32, from the group's X
 // tile in LDS (f16, rows of 144 bytes: no bank conflicts).
 //
-// What bounds it: instruction issue.  One wave issues a vector instruction
+// What bounds it: instruction issue, and with few stages per group the first
+// loads and the exchange at the end.  One wave issues a vector instruction
 // every 8 cycles and two waves on a SIMD one every 4 (measured on MI355X),
 // and an MFMA takes 32, so each SIMD needs two waves with at most about six
 // other instructions per MFMA; the weights of stage s + 1 and its X words
@@ -69,14 +89,17 @@ template <typename D, int XT, int YT, int TB, int RG, int KG, int PFW>
 DEV void gemm_group(const void* __restrict__ x, const uint8_t* __restrict__ w, void* __restrict__ y, int m,
                           int n, int k, int ldy, const GemmExt& ext) {
     // 32-row tiles per wave: one; more rows go to more workgroups (two leave
-    // too few registers for two waves per SIMD)
+    // too few registers for two waves per SIMD).  The arrays of one stay
+    // arrays: with scalars and references in their place the compiler spills
+    // the ring of raw weights (measured on MI355X, 64 x 128 tiles, Q4_K: 2.3
+    // times the time).
     constexpr int RA = 1;
     constexpr int BK = 64, KP = BK + 8;          // stage depth and LDS pitch (halves)
     constexpr int T = 32 * TB, BM = 32 * RA * RG;
     constexpr int NT = 64 * RG;                  // threads of a k group
     constexpr int ES = XT == XT_F32 ? 4 : 2, V = 16 / ES, LR = BK / V, RPI = NT / LR, NL = T / RPI;
     static_assert(T % RPI == 0 && NL >= 1, "x tile");
-    constexpr int NS = 4 * TB, NP = 8 * RA;      // slots (RA MFMAs each) and weight parts per stage
+    constexpr int NS = 4 * TB;                   // slots (RA MFMAs each) per stage
     constexpr int XBYTES = KG * 2 * T * KP * 2;
     constexpr int RBYTES = (KG - 1) * BM * T * 4;
     constexpr int LBYTES = XBYTES > RBYTES ? XBYTES : RBYTES;
@@ -118,23 +141,7 @@ DEV void gemm_group(const void* __restrict__ x, const uint8_t* __restrict__ w, v
         xr[p] = __builtin_bit_cast(
             uint4, __builtin_amdgcn_raw_buffer_load_b128(xrs, (int)xoff[p], stage_of(i) * (BK * ES), 0));
     };
-    auto xstore = [&](int p, int buf) INL {
-        uint16_t* dst = xl + buf * (T * KP) + xls + p * (RPI * KP);
-        const uint32_t v[4] = {xr[p].x, xr[p].y, xr[p].z, xr[p].w};
-        if constexpr (XT == XT_F16) {
-            *reinterpret_cast<uint4*>(dst) = make_uint4(v[0], v[1], v[2], v[3]);
-        } else if constexpr (XT == XT_BF16) {
-            uint32_t o[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                o[e] = pack_f16(__builtin_bit_cast(float, v[e] << 16), __builtin_bit_cast(float, v[e] & 0xffff0000u));
-            *reinterpret_cast<uint4*>(dst) = make_uint4(o[0], o[1], o[2], o[3]);
-        } else {
-            *reinterpret_cast<uint2*>(dst) =
-                make_uint2(pack_f16(__builtin_bit_cast(float, v[0]), __builtin_bit_cast(float, v[1])),
-                           pack_f16(__builtin_bit_cast(float, v[2]), __builtin_bit_cast(float, v[3])));
-        }
-    };
+    auto xstore = [&](int p, int buf) INL { store_x<XT>(xl + buf * (T * KP) + xls + p * (RPI * KP), xr[p]); };
 
     float16_t acc[RA][TB];
     static_for<RA * TB>([&](auto I) INL { acc[decltype(I)::value / TB][decltype(I)::value % TB] = float16_t{}; });
@@ -284,12 +291,14 @@ DEV void gemm_group(const void* __restrict__ x, const uint8_t* __restrict__ w, v
 // 16-k step are spread between the MFMAs, and the one barrier per stage
 // stands before its last step, whose fragments are already in registers.
 //
-// Bound by instruction issue as the group tiles are: 5.4 (Q8_0, f16 X) to
-// 10 (Q4_K, bf16 X) instructions per MFMA, against 28 us of MFMAs at 512
-// tokens on 14336x4096.  Measured on MI355X (14336x4096, cold, us) against
+// Bound by instruction issue where decoding is dear (Q4_K, bf16 X, 512
+// tokens: 7.8 vector instructions per MFMA, 0.46 of the SIMDs' time their
+// issue, 0.34 MFMAs); Q8_0 with f16 X (3.7 per MFMA) by the rounds of
+// workgroups: at 2048 tokens on 14336 rows 448 tiles on 256 CUs take two, with
+// MFMAs 0.51 of the time.  Measured on MI355X (14336x4096, cold, us) against
 // 128 x 128 and 128 x 256 tiles of four waves: Q4_K, bf16 X: 512 tokens
-// 109 -> 76 (128 x 256), 2048 tokens 400 -> 260 (256 x 256; 128 x 256: 299);
-// Q8_0, f16 X: 122 -> 72 and 440 -> 240.
+// 100 -> 73 (128 x 256), 2048 tokens 400 -> 260 (256 x 256; 128 x 256: 299);
+// Q8_0, f16 X: 122 -> 72 and 434 -> 245.
 template <typename D, int XT, int YT, int RA, int TB, int WR, int WC>
 DEV void gemm_wide(const void* __restrict__ x, const uint8_t* __restrict__ w, void* __restrict__ y, int m, int n,
                    int k, int ldy, const GemmExt& ext) {
@@ -309,7 +318,7 @@ DEV void gemm_wide(const void* __restrict__ x, const uint8_t* __restrict__ w, vo
     const size_t row_bytes = (size_t)(k / D::BE) * D::BB;
     const auto dc = D::ctx(w, ext);
     fmt_init<D>(dc, ext);
-    const int nk = k / BK, nsub = k / 32, nu = (nk + U - 1) / U;
+    const int nk = k / BK, nsub = k / 32;
 
     XScan<XT, NT> xscan;
 
@@ -330,23 +339,7 @@ DEV void gemm_wide(const void* __restrict__ x, const uint8_t* __restrict__ w, vo
         xr[P] = __builtin_bit_cast(
             uint4, __builtin_amdgcn_raw_buffer_load_b128(xrs, (int)xoff[P], min(s, nk - 1) * (BK * ES), 0));
     };
-    auto xstore = [&](auto P, int buf) INL {
-        uint16_t* dst = &xl[buf][xst + P * (RPI * XP)];
-        const uint32_t v[4] = {xr[P].x, xr[P].y, xr[P].z, xr[P].w};
-        if constexpr (XT == XT_F16) {
-            *reinterpret_cast<uint4*>(dst) = make_uint4(v[0], v[1], v[2], v[3]);
-        } else if constexpr (XT == XT_BF16) {
-            uint32_t o[4];
-            static_for<4>([&](auto E) INL {
-                o[E] = pack_f16(__builtin_bit_cast(float, v[E] << 16), __builtin_bit_cast(float, v[E] & 0xffff0000u));
-            });
-            *reinterpret_cast<uint4*>(dst) = make_uint4(o[0], o[1], o[2], o[3]);
-        } else {
-            *reinterpret_cast<uint2*>(dst) =
-                make_uint2(pack_f16(__builtin_bit_cast(float, v[0]), __builtin_bit_cast(float, v[1])),
-                           pack_f16(__builtin_bit_cast(float, v[2]), __builtin_bit_cast(float, v[3])));
-        }
-    };
+    auto xstore = [&](auto P, int buf) INL { store_x<XT>(&xl[buf][xst + P * (RPI * XP)], xr[P]); };
 
     float16_t acc[RA][TB];
     static_for<NM>([&](auto I) INL { acc[I / TB][I % TB] = float16_t{}; });
@@ -385,7 +378,6 @@ DEV void gemm_wide(const void* __restrict__ x, const uint8_t* __restrict__ w, vo
     // unit u + 1, decoded into the other buffer meanwhile.
     auto unit = [&](int u, auto WB, typename D::Raw& nxt) INL {
         constexpr int wb = decltype(WB)::value;
-        constexpr int FPS = 1;
         constexpr int NSLOT = U * 4 * NM, LAST = NSLOT - NM;  // slots; weights are in LDS before the last step
         const int jn = sub_of(u + 1);
         const typename D::P pr = D::prep(dc, nxt, wp, jn);
@@ -398,17 +390,13 @@ DEV void gemm_wide(const void* __restrict__ x, const uint8_t* __restrict__ w, vo
             if constexpr (q == 3) __syncthreads();
             static_for<NM>([&](auto I) INL {
                 constexpr int i = decltype(I)::value, a = i / TB, b = i % TB, slot = qq * NM + i;
-                // fragments of the next step, FPS a slot from this one's start
-                constexpr int f0 = i * FPS < RA + TB ? i * FPS : RA + TB;
-                constexpr int f1 = (i + 1) * FPS < RA + TB ? (i + 1) * FPS : RA + TB;
-                static_for<f1 - f0>([&](auto G) INL {
-                    constexpr int f = f0 + decltype(G)::value;
-                    std::integral_constant<int, f> F;
+                // a fragment of the next step a slot, from this one's start
+                if constexpr (i < RA + TB) {
                     std::integral_constant<int, set ^ 1> S;
-                    if constexpr (q < 3) frag(F, S, wb, xb, c, q + 1);
-                    else if constexpr (c + 1 < U) frag(F, S, wb, xb ^ 1, c + 1, 0);
-                    else frag(F, S, wb ^ 1, xb ^ 1, 0, 0);
-                });
+                    if constexpr (q < 3) frag(I, S, wb, xb, c, q + 1);
+                    else if constexpr (c + 1 < U) frag(I, S, wb, xb ^ 1, c + 1, 0);
+                    else frag(I, S, wb ^ 1, xb ^ 1, 0, 0);
+                }
                 acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[set][a], fb[set][b], acc[a][b], 0, 0, 0);
                 // weight parts due: eight over the slots before the last step
                 constexpr int p0 = slot < LAST ? slot * 8 / LAST : 8, p1 = slot < LAST ? (slot + 1) * 8 / LAST : 8;

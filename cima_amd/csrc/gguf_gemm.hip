@@ -1,5 +1,9 @@
 #include "gemm_tile.h"
 
+// X range flags (XRange in gemm_decode.h), for every kernel of this code object
+// and the 256 x 256 tiles'
+__device__ unsigned cima_gemm_status;
+
 // ------------------------------------------------------- prefill GEMM (MFMA)
 //
 // Y[m, n] (row stride ldy) = X[m, k] . W[n, k]^T: X holds m tokens, W is the
@@ -304,8 +308,8 @@ GEMM_SMALL(XT_BF16, bf16, XT_F16, f16)
 
 
 // Y[tok, row] (row stride ldy) = sum over z < S of part[z][tok][row], z in
-// order: the k-split partial tiles of the 16-token kernels, added in one
-// fixed order (results do not depend on the launch)
+// order: the k-split partial tiles, added in one fixed order (results do not
+// depend on the launch)
 template <int YT>
 __device__ void ksum_body(const float* __restrict__ part, void* __restrict__ y, int m, int n, int ldy, int S) {
     const long long o = (long long)blockIdx.x * 256 + threadIdx.x;

@@ -231,7 +231,9 @@ int cima_hip_gguf_gemm(cima_hip_ctx* ctx, int ggml_type, const void* x, const vo
  * partial tiles (S x m x n fp32, S = 2 or 4) in the slab (256-byte aligned)
  * and summed into Y in a fixed order by a second launch; without room in
  * the slab the call runs unsplit.  The slab's contents are then scratch:
- * calls that share a slab must not overlap. */
+ * calls that share a slab must not overlap, at any token count (callers on
+ * several streams pass a slab each, or slab_bytes 0: unsplit, and no slab
+ * is written). */
 int cima_hip_gguf_gemm_slab(cima_hip_ctx* ctx, int ggml_type, const void* x, const void* w, void* y,
                             int m, int n, int k, int ldy, int x_dtype, int y_dtype, void* slab,
                             unsigned long long slab_bytes);
