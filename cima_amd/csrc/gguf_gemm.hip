@@ -28,8 +28,8 @@ __device__ unsigned cima_gemm_status;
 //
 // Bound by memory round trips, with one or two stages in flight per wave, so
 // the order of a stage's instructions counts.  SER: weights and X by
-// SerialDeq and f2h2.  EARLY: the loads of the stage after next go out
-// before the barrier of this one.
+// SerialDeq and f2h2.  EARLY: the loads of the stage PF on go out before the
+// barrier of this one.
 template <typename D, int XT, int YT, int PF, int RT, bool SER, bool EARLY>
 __device__ void gemm_body_sk16(const void* __restrict__ x, const uint8_t* __restrict__ w, void* __restrict__ y,
                                int m, int n, int k, int ldy, const GemmExt& ext) {
