@@ -958,16 +958,18 @@ struct GemmTune {
 // stages (four 128-k stages, one per wave, for the 16-token tiles).
 //
 // Up to 32 tokens the estimates lie closer together than they are exact, so
-// a 16-token plan by the CUs' fill stands unless the cheapest is estimated 12 %
+// a 16-token plan by the CUs' fill stands unless the cheapest is estimated 7 %
 // below it: 16-row tiles where 32-row ones would fill at most half the CUs,
 // split four ways at a quarter workgroup per CU and two ways at a half;
-// 32-row ones split two ways at one; no split up to 2048 k, where the summing
-// launch costs more than it saves (Q4_K, bf16 X, 16 tokens: 512x2048 6.06
-// whole / 6.60 in four, 2048x2048 6.33 / 7.30 in two, but 1024x4096 9.05 /
-// 7.92 in four).  Over the 1092 runs short_cost is fitted to, us summed:
-// this choice is 9 % below the fill's plan on average and 2 % above the best;
-// by the estimate alone 13 runs were over 6 % above the fill's plan, with the
-// margin 3.
+// 32-row ones split two ways at one; no split below 4096 k (16-row tiles) or
+// 5120 (32-row), where the summing launch costs more than it saves (split
+// against whole, all formats and X types: 16-row tiles, four ways, k 2560
+// 1.04, 4096 0.80, 8192 0.59; 32-row, k 3584 1.22, 5120 0.99, 11008 0.89).
+// Over 2712 runs (30 weights, 3 to 32 tokens, the 1092 that short_cost is
+// fitted to among them) this choice is 1.5 % above the best plan on
+// average, by estimates fitted to Q4_K alone 5.4 %; of the 1092, 14 are over
+// 3 % slower than with the 16-token tiles and the rule before these, at most 7
+// %, and the mean is 20 % below.
 GemmPlan plan_gemm(const GemmTune& tune, int num_cu, int m, int n, int k, int x_dtype, const char* fname,
                    size_t part_bytes) {
     const int cu = num_cu > 0 ? num_cu : 1;
@@ -1018,12 +1020,12 @@ GemmPlan plan_gemm(const GemmTune& tune, int num_cu, int m, int n, int k, int x_
         const int wgs32 = (int)plan_wgs(GemmPlan{KB16, 1}, m, n, x_dtype);
         GemmPlan fill{2LL * wgs32 <= cu ? KB16N : KB16, 1};
         const int wgs = (int)plan_wgs(fill, m, n, x_dtype);
-        if (k <= 2048) fill.ksplit = 1;
+        if (k < (fill.kind == KB16 ? 5120 : 4096)) fill.ksplit = 1;
         else if (fill.kind == KB16) fill.ksplit = wgs <= cu ? 2 : 1;
         else fill.ksplit = 4 * wgs <= cu ? 4 : (2 * wgs <= cu ? 2 : 1);
         if (tune.ksplit) fill.ksplit = fits(fill.kind, tune.ksplit) ? tune.ksplit : 1;
         while (!fits(fill.kind, fill.ksplit)) fill.ksplit /= 2;
-        best = fill, best_t = 0.88 * cost(fill);
+        best = fill, best_t = 0.93 * cost(fill);
         if (!strcmp(fname, "f16w")) return best;
         consider(KB16);
         consider(KB16N);
