@@ -163,11 +163,27 @@ const char* const kModuleFiles[NUM_MODULES] = {"cima_gemv_a.hsaco", "cima_gemv_b
                                                "cima_gemm.hsaco",   "cima_dequant.hsaco", "cima_decode.hsaco",
                                                "cima_bnb4.hsaco",   "cima_gemm_wide.hsaco"};
 
-// weights and X types with _b16l_ kernels, the 32 x 16 prefill tiles for grids
-// of at most one workgroup per CU (sk16_serial in gguf_gemm.hip)
+// weights and X types whose 32 x 16 prefill tiles are built twice: _b16_ decodes
+// in one go, _b16l_ in parts (sk16_serial in gguf_gemm.hip)
 bool gemm_b16l(const char* weights, const char* xt) {
-    return !strcmp(weights, "q4_k") || !strcmp(weights, "q5_k") || !strcmp(weights, "iq4_xs") ||
-           (!strcmp(weights, "nf4") && !strcmp(xt, "f16"));
+    return strcmp(xt, "f32") && (!strcmp(weights, "q4_k") || !strcmp(weights, "q5_k") || !strcmp(weights, "iq4_xs") ||
+                                 (!strcmp(weights, "nf4") && !strcmp(xt, "f16")));
+}
+
+// Which of them runs (true: _b16_, in one go), by the workgroups per CU.  In
+// parts three share a CU, in one go two, so that three or five to a CU take a
+// round less in parts; at two or four the rounds are the same, and where X's
+// rows lie a multiple of 4 KB apart decoding in one go is the faster.  Measured
+// on MI355X, cold, us, in parts / in one go: Q4_K, bf16 X, 16 tokens:
+// 14336x4096 (2) 16.8 / 16.5, 18944x3584 (3) 21.8 / 23.3, 28672x4096 (4) 35.8 /
+// 32.6; 2 tokens 18944x3584 19.0 / 22.5; Q5_K 14336x4096 28.2 / 25.7; NF4, f16
+// X, 2 tokens 18944x3584 18.4 / 24.3, 16 tokens 28672x4096 (4) 32.2 / 30.0;
+// IQ4_XS 8192x4096 (1) 11.2 / 12.5.  Over 2700 products (9 heights, 10 k, 2 to
+// 32 tokens) 0.4 % above the better of the two on average, in parts
+// throughout 0.7 %, in one go 4.3 %.
+bool b16_serial(const char* weights, int k, long long per_cu) {
+    if (!strcmp(weights, "nf4")) return per_cu == 4;
+    return k % 2048 == 0 && (per_cu == 2 || (per_cu == 4 && strcmp(weights, "iq4_xs")));
 }
 
 // decode-step kernels (cima_decode.hsaco)
@@ -1076,7 +1092,8 @@ int gemm_launch(cima_hip_ctx* ctx, const char* fname, const void* x, const void*
     // a split group tile writes fp32 partial tiles through its Y
     const bool part_y = ks > 1 && !sk;
     const unsigned gx = (unsigned)((n + bm - 1) / bm), gy = (unsigned)((m + bn - 1) / bn);
-    const bool low = p.kind == KB16 && (long long)gx * gy * ks <= ctx->num_cu && gemm_b16l(fname, xn[x_dtype]);
+    const long long per_cu = ((long long)gx * gy * ks + ctx->num_cu - 1) / std::max(ctx->num_cu, 1);
+    const bool low = p.kind == KB16 && gemm_b16l(fname, xn[x_dtype]) && !b16_serial(fname, k, per_cu);
     char name[96];
     snprintf(name, sizeof name, "cima_gemm_%s_%s_%s_%s", fname, low ? "b16l" : kn[p.kind], xn[x_dtype],
              y_dtype == CIMA_DT_F32 || part_y ? "f32" : "f16");

@@ -173,18 +173,16 @@ constexpr int group_occ() { return BN == 32 && XT != XT_F32 && sizeof(typename D
 template <int BN, int XT>
 constexpr int group_rg() { return BN == 128 && XT == XT_F32 ? 4 : 2; }
 
-// 32-row 16-token tiles with SerialDeq where several workgroups share a CU
-// (measured on MI355X, cold, us, part() / SerialDeq: Q4_K, bf16 X, 14336x4096
-// at 16 tokens 17.7 / 17.3, 28672x4096 35.8 / 32.6; Q5_K 28.2 / 25.7 and 52.8 /
-// 48.4; IQ4_XS 17.5 / 16.6; NF4, f16 X, 28672x4096 32.2 / 30.0); the other
-// formats are no faster that way (Q4_1 16.1 / 16.2, Q5_1 16.3 / 18.1, NF4,
-// bf16 X, 16.3 / 21.9), and nor is a grid of at most one workgroup per CU,
-// which for these formats has kernels of its own, _b16l_ (8192x4096: Q4_K
-// 12.7 / 12.9, IQ4_XS 11.2 / 12.5, Q5_K 17.7 / 18.7).
+// 32-row 16-token tiles built with SerialDeq, and with part() as _b16l_; which
+// one runs follows from k and the workgroups per CU (b16_serial in
+// cima_hip.cpp).  part() lets three workgroups share a CU, SerialDeq two.
+// The other formats, and f32 X, are no faster with SerialDeq (measured on
+// MI355X, 14336x4096 at 16 tokens, cold, us, part() / SerialDeq: Q4_1 16.1 /
+// 16.2, Q5_1 16.3 / 18.1, NF4, bf16 X, 16.3 / 21.9).
 template <typename D, int XT>
 constexpr bool sk16_serial() {
-    return std::is_same<D, GG<DQ4_K>>::value || std::is_same<D, GG<DQ5_K>>::value ||
-           std::is_same<D, GG<DIQ4_XS>>::value || (std::is_same<D, DNF4>::value && XT == XT_F16);
+    return XT != XT_F32 && (std::is_same<D, GG<DQ4_K>>::value || std::is_same<D, GG<DQ5_K>>::value ||
+                            std::is_same<D, GG<DIQ4_XS>>::value || (std::is_same<D, DNF4>::value && XT == XT_F16));
 }
 
 // name: cima_gemm_<fmt>_b<BN>_<x type>_<y type>
@@ -251,7 +249,7 @@ constexpr int sk16n_pf() {
         gemm_body_sk16<D, XT, YT, 1, 2, false, false>(x, w, y, m, n, k, ldy, ext);                  \
     }
 #define GEMM_XY_LOW(FN, D, XT, XN) GEMM_KERNEL_LOW(FN, D, XT, XN, XT_F32, f32) GEMM_KERNEL_LOW(FN, D, XT, XN, XT_F16, f16)
-#define GEMM_LOW(FN, D) GEMM_XY_LOW(FN, D, XT_F32, f32) GEMM_XY_LOW(FN, D, XT_F16, f16) GEMM_XY_LOW(FN, D, XT_BF16, bf16)
+#define GEMM_LOW(FN, D) GEMM_XY_LOW(FN, D, XT_F16, f16) GEMM_XY_LOW(FN, D, XT_BF16, bf16)
 #define GEMM_FMT(FN, D) \
     GEMM_XY(FN, D, 16) GEMM_XY_NARROW(FN, D) GEMM_XY(FN, D, 32) GEMM_XY(FN, D, 64) GEMM_XY(FN, D, 128) GEMM_XY(FN, D, 256)
 

@@ -65,7 +65,7 @@ def test_code_object_holds_every_kernel():
                     if bn == 16:
                         assert f"cima_gemm_{f}_b16n_{xt}_{yt}".encode() in blobs["gemm"]
                         low = f"cima_gemm_{f}_b16l_{xt}_{yt}".encode() in blobs["gemm"]
-                        assert low == (f in ("q4_k", "q5_k", "iq4_xs"))
+                        assert low == (f in ("q4_k", "q5_k", "iq4_xs") and xt != "f32")
 
 
 def test_stream_read_kernel_present():
@@ -238,10 +238,10 @@ def test_gemm_kernels_do_not_spill():
     compiler does not promote -- turns each stage into scratch traffic)."""
     notes = _kernel_notes(cbuild.HSACOS["gemm"])
     # nine GGUF formats, bitsandbytes 4-bit and f16 weights: six tile kinds
-    # x six (x, y) dtype pairs each, the 16-token tiles of low grids (three
-    # formats, and NF4 for f16 X), plus the six plain f16-weight kernels and
-    # the two k-split sums
-    assert len(notes) == 11 * 6 * 6 + 3 * 6 + 2 + 6 + 2
+    # x six (x, y) dtype pairs each, the 32 x 16 tiles built twice (three formats
+    # for f16 and bf16 X, and NF4 for f16 X), plus the six plain f16-weight
+    # kernels and the two k-split sums
+    assert len(notes) == 11 * 6 * 6 + 3 * 4 + 2 + 6 + 2
     # the 256 x 256 tiles, not built for f32 X
     wide = _kernel_notes(cbuild.HSACOS["gemm_wide"])
     assert len(wide) == 11 * 2 * 2

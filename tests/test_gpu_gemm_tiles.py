@@ -236,12 +236,13 @@ def test_planned_k_split_of_the_wide_group_tiles(hip, t, m, n, k, xd, plan):
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q5_K, IQ4_XS, 0], ids=["q4_k", "q5_k", "iq4_xs", "nf4"])
-@pytest.mark.parametrize("k", [256, 768, 1280])
-def test_32_row_tiles_of_full_and_low_grids(hip, t, k):
-    """The 16-token tiles decode in one way where several workgroups share a
-    CU (257 row tiles here) and in another below (slices of 4096 rows, at
-    most 128 tiles): the same bits, at 2, 6 and 10 stages."""
-    n, m, bs = 8225, 13, 64
+@pytest.mark.parametrize("n, k", [(8225, 256), (8225, 768), (8225, 1280), (8225, 2048), (24617, 2048)])
+def test_32_row_tiles_of_full_and_low_grids(hip, t, n, k):
+    """The 32-row tiles decode in one go at two and four workgroups per CU
+    where k is a multiple of 2048 (258 and 770 row tiles; NF4 at four, any k)
+    and in parts otherwise (slices of 4096 rows, at most 128 tiles): the same
+    bits."""
+    m, bs = 13, 64
     rng = np.random.default_rng(k)
     if t:
         w = torch.from_numpy(synth.weights(t, 300 + t, 0.02, n, k).reshape(n, -1)).cuda()
